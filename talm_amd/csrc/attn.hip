@@ -7,9 +7,9 @@
 // reference's per-KV-head memory-efficient attention launches (solution/unpad.py:199-294), whose
 // semantics are per-row causal SDPA (solution/unpad.py:121-134).
 //
-// The forward is a flash-attention pass per (sequence, 32-row query tile, query heads of one KV
-// head), its key tiles of 64 split between two groups of wavefronts and streamed with
-// direct-to-LDS loads. Scores are computed transposed, S^T = K Q^T (v_mfma_f32_32x32x16_f16), so
+// The forward is a flash-attention pass per (sequence, query tile, query heads of one KV head),
+// 32 query rows of a head per wavefront, its key tiles of 64 streamed with direct-to-LDS loads and,
+// where few workgroups leave the chip idle, split between two groups of wavefronts. Scores are computed transposed, S^T = K Q^T (v_mfma_f32_32x32x16_f16), so
 // each lane owns one query row (its accumulator column): the online max / sum and the output
 // rescale are per-lane scalars. The exponentiated scores are already in the B-operand layout of
 // O^T = V^T P^T: the reduction over keys takes the accumulator's key order as its k-slot order,
@@ -47,6 +47,15 @@ constexpr float kLn2 = 0.693147180559945309f;
 
 __device__ __forceinline__ float exp2_(float x) { return __builtin_amdgcn_exp2f(x); }
 
+// The larger of lane l's and lane l ^ 32's value (v_permlane32_swap: the first result holds the
+// lower half's values in both halves, the second the upper half's).
+__device__ __forceinline__ float half_max(float x) {
+  const uint32_t u = __builtin_bit_cast(uint32_t, x);
+  const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  const uint32_t lo = r[0], hi = r[1];
+  return fmaxf(__builtin_bit_cast(float, lo), __builtin_bit_cast(float, hi));
+}
+
 struct FwdArgs {
   const uint16_t* q;
   int64_t q_tok, q_head;
@@ -57,7 +66,7 @@ struct FwdArgs {
   const int32_t* cu;
   int group;          // query heads per KV head
   int head_chunks;    // workgroups per KV head (group / heads per workgroup)
-  int n_tiles;        // 32-row query tiles per sequence (of the longest)
+  int rank_x;         // the grid's axes: (chunk, sequence, rank), or (rank, chunk, sequence)
   float scale_log2;   // softmax scale * log2(e)
   uint16_t* out;
   int64_t o_tok, o_head;
@@ -108,6 +117,29 @@ __device__ __forceinline__ void read_tr_operand_untracked(const unsigned char* t
   lo = read_tr_untracked(tile + tile_chunk(row, col >> 3) * 16 + (col & 7) * 2);
   hi = read_tr_untracked(tile + tile_chunk(row + 8, col >> 3) * 16 + (col & 7) * 2);
 }
+// The same at an LDS address plus a constant offset, and a 16-byte read likewise.
+__device__ __forceinline__ uint32_t lds_addr(const unsigned char* lds) {
+  return static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
+      (__attribute__((address_space(3))) const unsigned char*)(lds)));
+}
+__device__ __forceinline__ half4_t read_tr_untracked(uint32_t addr, int off) {
+  half4_t r;
+  asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(r) : "v"(addr), "n"(off));
+  return r;
+}
+__device__ __forceinline__ half8_t read16_untracked(uint32_t addr, int off) {
+  half8_t r;
+  asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(r) : "v"(addr), "n"(off));
+  return r;
+}
+// Wait until at most n LDS operations are in flight (they return in order); the registers count
+// as rewritten here.
+__device__ __forceinline__ void lgkm_wait(int n, half8_t& r) {
+  asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(r) : "n"(n));
+}
+__device__ __forceinline__ void lgkm_wait(int n, half4_t& r, half4_t& q) {
+  asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(r), "+v"(q) : "n"(n));
+}
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ f32x4_t read_f4_untracked(const float* lds) {
   const uint32_t addr = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
@@ -156,41 +188,97 @@ __device__ __forceinline__ void dma_tile(const uint16_t* base, int64_t ld, int r
   }
 }
 
-// Forward, one workgroup per (sequence, 32-row query tile, W query heads of one KV head), with
-// S groups of W wavefronts: group g takes the key tiles g, g + S, g + 2 S, ..., one wavefront per
-// head, so the serial key loop of a long query tile is S times shorter (its length, not the
-// chip, bounds the kernel at these sequence lengths); the groups' partial results are merged
-// through LDS at the end. The K / V tiles of the KV head are loaded once for the W heads.
+// dma_tile with the per-lane part formed once, in one register: the lane's byte offset in block
+// `wave`. Block wave + W * it lies 4 W it rows on (a multiple of 16 for W = 4, so its swizzle is
+// the same), which the load takes as its scalar offset.
+struct TileDma {
+  static constexpr int W = 4, kPer = kKeys / 4 / W;
+  uint32_t off, step;  // step: bytes of 4 W rows (scalar)
+  int row;
+  __device__ __forceinline__ void init(int64_t ld, int wave, int lane) {
+    row = 4 * wave + (lane >> 4);
+    off = static_cast<uint32_t>((row * ld + ((lane & 15) ^ tile_swz(row)) * 8) * 2);
+    step = static_cast<uint32_t>(4 * W * ld * 2);
+  }
+  __device__ __forceinline__ void issue(const uint16_t* base, int rows_valid, unsigned char* dst,
+                                        int wave) const {
+    const __amdgpu_buffer_rsrc_t rsrc = buffer_rsrc(base);
+#pragma unroll
+    for (int it = 0; it < kPer; ++it)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr_t)(dst + (wave + it * W) * 1024), 16,
+                                               row + 4 * W * it < rows_valid ? off : kOob, it * step, 0, 0);
+  }
+};
+
+// Runs body(tile, slot) for tile = 0 .. n - 1 in ring slot tile & 1, after issue(tile + 1, slot)
+// put the next tile in flight into the other slot. Each tile's loads are waited for (this
+// wavefront's, then the barrier for everyone's) right before its body, and the barrier also
+// retires the slot the previous body read. Unrolled by two, so every slot address is a
+// compile-time offset. (A third slot, two tiles in flight, measured slower.)
+template <class Issue, class Body>
+__device__ __forceinline__ void ring2(int n, Issue&& issue, Body&& body) {
+  issue(0, 0);
+  for (int t = 0; t < n; t += 2) {
+    wait_vmcnt<0>();
+    lds_barrier();
+    if (t + 1 < n) issue(t + 1, 1);
+    body(t, 0);
+    if (t + 1 >= n) break;
+    wait_vmcnt<0>();
+    lds_barrier();
+    if (t + 2 < n) issue(t + 2, 0);
+    body(t + 1, 1);
+  }
+}
+
+// Forward, one workgroup per (sequence, H query heads of one KV head, 32 * (4 / H) query rows):
+// S groups of four wavefronts, each wavefront a head and 32 query rows, group g the key tiles g,
+// g + S, ... of 64 keys through a two-slot ring of its own.
 // Scores are computed transposed, S^T = K Q^T, so each lane owns one query row: the online
 // max / sum and the output rescale are per-lane scalars, and the exponentiated scores are
 // already the B operand of O^T = V^T P^T, whose A operand is read transposed from the row-major
-// V tile. Two LDS slots per group: the next tiles' loads fly during this step's math.
-template <int W, int S>
-__global__ __launch_bounds__(64 * W * S) void attn_fwd_kernel(FwdArgs a) {
-  constexpr int kStepBytes = S * 2 * kTileBytes;        // the K and V tiles of one step
-  constexpr int kRing = 2 * kStepBytes;
-  constexpr int kMerge = (S - 1) * W * (64 * 64 * 4 + 64 * 8);  // partial O, m, l per wavefront
-  constexpr int kStage = W * 32 * kKS * 2;              // fp16 output rows per head
-  constexpr int kSmem = kRing > kMerge + kStage ? kRing : kMerge + kStage;
-  __shared__ __attribute__((aligned(1024))) unsigned char smem[kSmem];
+// V tile.
+// S = 1 where the grid fills the chip: two workgroups share a CU (64 KiB of LDS and at most 256
+// registers each), so the two wavefronts of a SIMD belong to different workgroups and no barrier
+// keeps them in step: one's softmax runs on the VALU while the other has the matrix core. What
+// bounds it then: the clock, which falls from 2.4 to about 1.4 GHz with the matrix cores and the
+// VALU busy together (a probe's MFMA + exponential loop), and the K / V reads from LDS.
+// Against one workgroup of six or eight wavefronts per CU on 32 query rows (128 KiB of LDS, K
+// operands waited for one by one): 16 rows of 128..512 tokens 36.2 -> 19.9 us, 16 of 1..1024 72.4 ->
+// 39.3, [4096, 3001, 2222, 1531] 187 -> 132 us (543 -> 769 TF/s), config 2's four rows 13.7 -> 13.0.
+// Not kept: the next tile's S^T issued between this one's exponentials and P V (127 against 119 us
+// for 8 rows of 2048: 253 registers, the same clock), s_setprio around the MFMAs (no change).
+// S = 2 where it does not: the longest workgroup's chain of key tiles sets the time (about 1.1 us
+// per tile), and two groups halve it; their partial results are merged through LDS at the end.
+template <int H, int S>
+__global__ __launch_bounds__(256 * S, 2) void attn_fwd_kernel(FwdArgs a) {
+  constexpr int R = 4 / H;           // 32-row blocks per workgroup
+  constexpr int kRows = 32 * R;
+  constexpr int kSlot = 2 * kTileBytes;  // one step's K and V tiles
+  constexpr int kRing = 2 * kSlot;       // of one group
+  constexpr int kStage = 4 * 32 * kKS * 2;  // fp16 output rows
+  constexpr int kMerge = (S - 1) * 4 * (64 * 64 * 4 + 64 * 8);  // partial O, m, l per wavefront
+  static_assert(S <= 2 && kMerge + kStage <= S * kRing, "merge and output staging reuse the rings");
+  __shared__ __attribute__((aligned(1024))) unsigned char smem[S * kRing];
 
-  const int seq = blockIdx.z;
-  const int kvh = static_cast<int>(blockIdx.y) / a.head_chunks;
-  const int hc = static_cast<int>(blockIdx.y) % a.head_chunks;
-  const int tile = a.n_tiles - 1 - static_cast<int>(blockIdx.x);  // longest tiles first
+  const int rank = static_cast<int>(a.rank_x ? blockIdx.x : blockIdx.z);
+  const int chunk = static_cast<int>(a.rank_x ? blockIdx.y : blockIdx.x);
+  const int seq = static_cast<int>(a.rank_x ? blockIdx.z : blockIdx.y);
+  const int kvh = chunk / a.head_chunks, hc = chunk % a.head_chunks;
   const int s0 = a.cu[seq], len = a.cu[seq + 1] - s0;
-  const int q0 = tile * 32;
-  if (q0 >= len) return;  // the whole workgroup, before any barrier
+  const int tile = (len + kRows - 1) / kRows - 1 - rank;  // every sequence's longest tiles first
+  if (tile < 0) return;  // the whole workgroup, before any barrier
+  const int q0 = tile * kRows;
   const int tid = threadIdx.x, lane = tid & 63;
   // the wavefront index in a scalar register: everything the branches, loop bounds and the
   // direct-to-LDS addresses derive from it stays wavefront-uniform
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int hw = wave % W, grp = wave / W;  // head slot, key group
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave = wid & 3, grp = wid >> 2;
   const int hh = lane >> 5, l32 = lane & 31;
-  const int head = kvh * a.group + hc * W + hw;
+  const int head = kvh * a.group + hc * H + wave % H;
+  const int w0 = q0 + 32 * (wave / H);  // the wavefront's first query row
 
-  // this lane's query row and its Q fragments (the B operand: k-slots d = 16 s + 8 hh .. + 8)
-  const int qrow = q0 + l32;
+  const int qrow = w0 + l32;
   const int qr = min(qrow, len - 1);
   half8_t qf[kD / 16];
   {
@@ -198,24 +286,21 @@ __global__ __launch_bounds__(64 * W * S) void attn_fwd_kernel(FwdArgs a) {
 #pragma unroll
     for (int s = 0; s < kD / 16; ++s) qf[s] = *reinterpret_cast<const half8_t*>(qp + 16 * s);
   }
-
-  const int kend = min(len, q0 + 32);  // keys any row of this tile can see
-  const int n_kt = (kend + kKeys - 1) / kKeys;
+  const int n_kt = (min(len, q0 + kRows) + kKeys - 1) / kKeys;
   const int n_steps = (n_kt + S - 1) / S;
-  const int key_lim = min(qrow, len - 1);  // the last key this lane's row may see
+  const int my_kt = (min(len, w0 + 32) + kKeys - 1) / kKeys;  // tiles the wavefront's rows see
   const uint16_t* kbase = a.k + static_cast<int64_t>(s0) * a.k_tok + kvh * a.k_head;
   const uint16_t* vbase = a.v + static_cast<int64_t>(s0) * a.v_tok + kvh * a.v_head;
-  // the group's W wavefronts load its tile: 16 blocks of 1 KiB per K or V tile, block b by
-  // wavefront b % W of the group
-  auto slot_of = [&](int step) { return smem + (step & 1) * kStepBytes + grp * 2 * kTileBytes; };
-  auto issue = [&](int step) {  // the group's tile of `step`, if it exists
+  TileDma kd, vd;
+  kd.init(a.k_tok, wave, lane);
+  vd.init(a.v_tok, wave, lane);
+  auto issue = [&](int step, int slot) {
     const int kt = step * S + grp;
-    if (kt >= n_kt) return;
-    unsigned char* slot = slot_of(step);
-    const int r0 = kt * kKeys;
-    dma_tile<W>(kbase + static_cast<int64_t>(r0) * a.k_tok, a.k_tok, len - r0, slot, hw, lane);
-    dma_tile<W>(vbase + static_cast<int64_t>(r0) * a.v_tok, a.v_tok, len - r0, slot + kTileBytes,
-                hw, lane);
+    if (S > 1 && kt >= n_kt) return;
+    unsigned char* dst = smem + grp * kRing + slot * kSlot;
+    kd.issue(kbase + static_cast<int64_t>(kt * kKeys) * a.k_tok, len - kt * kKeys, dst, wave);
+    vd.issue(vbase + static_cast<int64_t>(kt * kKeys) * a.v_tok, len - kt * kKeys, dst + kTileBytes,
+             wave);
   };
 
   f32x16 o[kD / 32];
@@ -230,54 +315,61 @@ __global__ __launch_bounds__(64 * W * S) void attn_fwd_kernel(FwdArgs a) {
   float m = -INFINITY, lsum = 0.f;
   const float c = a.scale_log2;
 
-  issue(0);
-  for (int step = 0; step < n_steps; ++step) {
+  // LDS addresses of the operand reads at slot 0 of the group's ring: K rows l32 of chunk 2 s + hh (s through an XOR
+  // of bits 5..7), V's transposing reads of column block j (bits 6, 7), rows 4 (lane / 32) + .. and
+  // 8 rows on
+  const uint32_t lds0 = lds_addr(smem) + grp * kRing;
+  uint32_t kaddr[kD / 16], vlo[kD / 32], vhi[kD / 32];
+#pragma unroll
+  for (int s = 0; s < kD / 16; ++s) kaddr[s] = lds0 + tile_chunk(l32, 2 * s + hh) * 16;
+  {
+    const int g = lane >> 4, i = lane & 15;
+#pragma unroll
+    for (int j = 0; j < kD / 32; ++j) {
+      const int col = 32 * j + 16 * (g & 1) + 4 * (i & 3), row = 4 * (g >> 1) + (i >> 2);
+      vlo[j] = lds0 + tile_chunk(row, col >> 3) * 16 + (col & 7) * 2;
+      vhi[j] = lds0 + tile_chunk(row + 8, col >> 3) * 16 + (col & 7) * 2;
+    }
+  }
+  auto body = [&](int step, auto slot_) __attribute__((always_inline)) {
+    constexpr int kOff = decltype(slot_)::value * kSlot;
     const int kt = step * S + grp;
-    // this group's tile of the step has landed (the next step's loads are not issued yet)
-    wait_vmcnt<0>();
-    lds_barrier();  // every group's tile has; everyone is done with step - 1 (its slots are free)
-    issue(step + 1);
-    if (kt >= n_kt) continue;  // this group has no tile left (barriers stay matched: no return)
-    const unsigned char* ks = slot_of(step);
-    const unsigned char* vs = ks + kTileBytes;
-    const uint4* k16 = reinterpret_cast<const uint4*>(ks);
+    if (kt >= my_kt) return;  // every key of the tile is after every row of the wavefront
     const int k0 = kt * kKeys;
-    // S^T for keys k0 + 32 b + (8 (v / 4) + 4 hh + v % 4), this lane's query column
+    // S^T: the second 32 keys' operand reads are issued one by one behind the first block's MFMAs
     f32x16 st[2];
+    half8_t kf[kD / 16];
+#pragma unroll
+    for (int s = 0; s < kD / 16; ++s) kf[s] = read16_untracked(kaddr[s], kOff);
 #pragma unroll
     for (int b = 0; b < 2; ++b) {
 #pragma unroll
       for (int v = 0; v < 16; ++v) st[b][v] = 0.f;
-      // the block's 8 operand reads issued before its MFMAs
-      half8_t ka[kD / 16];
 #pragma unroll
-      for (int s = 0; s < kD / 16; ++s)
-        ka[s] = __builtin_bit_cast(half8_t, k16[tile_chunk(32 * b + l32, 2 * s + hh)]);
-      __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);
-      __builtin_amdgcn_sched_group_barrier(0x008, 8, 0);
-#pragma unroll
-      for (int s = 0; s < kD / 16; ++s)
-        st[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ka[s], qf[s], st[b], 0, 0, 0);
+      for (int s = 0; s < kD / 16; ++s) {
+        lgkm_wait(b == 0 ? 7 : 7 - s, kf[s]);
+        st[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[s], qf[s], st[b], 0, 0, 0);
+        if (b == 0) {
+          __builtin_amdgcn_sched_barrier(0);
+          kf[s] = read16_untracked(kaddr[s], kOff + 8192);
+        }
+      }
     }
-    // causal / length mask only on a tile that reaches past the first query row of the
-    // workgroup or past the sequence: a real (uniform) branch; the empty volatile asm keeps the
-    // compiler from turning it into selects executed on every tile
-    if (k0 + kKeys - 1 > q0 || k0 + kKeys > len) {
+    if (k0 + kKeys - 1 > w0 || k0 + kKeys > len) {  // uniform: the diagonal and the last tile
+      const int lim = qr - k0 - 4 * hh;
       asm volatile("");
 #pragma unroll
       for (int b = 0; b < 2; ++b)
 #pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const int key = k0 + 32 * b + 8 * (v >> 2) + 4 * hh + (v & 3);
-          st[b][v] = key > key_lim ? -INFINITY : st[b][v];
-        }
+        for (int v = 0; v < 16; ++v)
+          st[b][v] = 32 * b + 8 * (v >> 2) + (v & 3) > lim ? -INFINITY : st[b][v];
     }
     float mt = -INFINITY;
 #pragma unroll
     for (int b = 0; b < 2; ++b)
 #pragma unroll
       for (int v = 0; v < 16; ++v) mt = fmaxf(mt, st[b][v]);
-    mt = c * fmaxf(mt, __shfl_xor(mt, 32, kWave));
+    mt = c * half_max(mt);
     const bool grow = mt > m + kLazy;
     if (__ballot(grow)) {  // some row's maximum moved: rescale those rows
       asm volatile("");
@@ -290,12 +382,13 @@ __global__ __launch_bounds__(64 * W * S) void attn_fwd_kernel(FwdArgs a) {
 #pragma unroll
         for (int v = 0; v < 16; ++v) o[j][v] *= alpha;
     }
-    // V^T operands of the four 16-key groups (b, h), read untracked two groups at a time
     half4_t vt[2][8];
-    auto read_v = [&](int grp16, int buf) {
+    auto read_v = [&](int g16, int buf) __attribute__((always_inline)) {
 #pragma unroll
-      for (int j = 0; j < kD / 32; ++j)
-        read_tr_operand_untracked(vs, 16 * grp16, 32 * j, lane, vt[buf][2 * j], vt[buf][2 * j + 1]);
+      for (int j = 0; j < kD / 32; ++j) {
+        vt[buf][2 * j] = read_tr_untracked(vlo[j], kOff + kTileBytes + g16 * 4096);
+        vt[buf][2 * j + 1] = read_tr_untracked(vhi[j], kOff + kTileBytes + g16 * 4096);
+      }
     };
     read_v(0, 0);
     float ps = 0.f;
@@ -308,7 +401,6 @@ __global__ __launch_bounds__(64 * W * S) void attn_fwd_kernel(FwdArgs a) {
         ps += pv;
       }
     lsum += ps;
-    // O^T[d][q] += V^T[d][key] P^T[key][q], 16 keys per step in the accumulator's key order
 #pragma unroll
     for (int g16 = 0; g16 < 4; ++g16) {
       const int b = g16 >> 1, h = g16 & 1, buf = g16 & 1;
@@ -324,33 +416,30 @@ __global__ __launch_bounds__(64 * W * S) void attn_fwd_kernel(FwdArgs a) {
                                                                 0, 1, 2, 3, 4, 5, 6, 7)),
             pb, o[j], 0, 0, 0);
     }
-  }
+  };
+  ring2(n_steps, issue, [&](int step, int slot) __attribute__((always_inline)) {
+    if (slot) body(step, std::integral_constant<int, 1>{});
+    else body(step, std::integral_constant<int, 0>{});
+  });
   lsum += __shfl_xor(lsum, 32, kWave);  // the row's sum over both halves of the lanes
-
-  // merge the groups into group 0: each other group's wavefront leaves its (m, l, O) in LDS
   __syncthreads();  // every wavefront is done with the tiles
-  float* part_o = reinterpret_cast<float*>(smem);                        // [group-1][W][64][64]
-  float* part_ml = part_o + (S - 1) * W * 64 * 64;                       // [group-1][W][64][2]
-  if (grp > 0) {
-    float* po = part_o + ((grp - 1) * W + hw) * 64 * 64;
+  if constexpr (S > 1) {  // group 1 leaves its (m, l, O) in LDS, group 0 merges
+    float* po = reinterpret_cast<float*>(smem) + wave * 64 * 64;
+    float* pml = reinterpret_cast<float*>(smem) + 4 * 64 * 64 + wave * 64 * 2;
+    if (grp > 0) {
 #pragma unroll
-    for (int j = 0; j < kD / 32; ++j)
+      for (int j = 0; j < kD / 32; ++j)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) po[(16 * j + v) * 64 + lane] = o[j][v];
-    float* pml = part_ml + ((grp - 1) * W + hw) * 64 * 2;
-    pml[2 * lane] = m;
-    pml[2 * lane + 1] = lsum;
-  }
-  __syncthreads();
-  if (grp > 0) return;  // no barrier follows for the other groups
-#pragma unroll
-  for (int g = 1; g < S; ++g) {
-    const float* po = part_o + ((g - 1) * W + hw) * 64 * 64;
-    const float* pml = part_ml + ((g - 1) * W + hw) * 64 * 2;
+        for (int v = 0; v < 16; ++v) po[(16 * j + v) * 64 + lane] = o[j][v];
+      pml[2 * lane] = m;
+      pml[2 * lane + 1] = lsum;
+    }
+    __syncthreads();
+    if (grp > 0) return;  // no barrier follows
     const float m2 = pml[2 * lane], l2 = pml[2 * lane + 1];
-    const float m_new = fmaxf(m, m2);
-    const float a1 = m == -INFINITY ? 0.f : exp2_(m - m_new);
-    const float a2 = m2 == -INFINITY ? 0.f : exp2_(m2 - m_new);
+    const float m_new = fmaxf(m, m2);  // m is finite: group 0 has key tile 0
+    const float a1 = exp2_(m - m_new);
+    const float a2 = exp2_(m2 - m_new);  // 0 when group 1 had no tile (m2 = -inf)
     m = m_new;
     lsum = lsum * a1 + l2 * a2;
 #pragma unroll
@@ -359,9 +448,9 @@ __global__ __launch_bounds__(64 * W * S) void attn_fwd_kernel(FwdArgs a) {
       for (int v = 0; v < 16; ++v) o[j][v] = o[j][v] * a1 + po[(16 * j + v) * 64 + lane] * a2;
   }
 
-  // O = O^T / l through LDS: each head stages its 32 rows x D, then 16-byte row stores
+  // O = O^T / l through LDS: each wavefront stages its 32 rows x D, then 16-byte row stores
   const float inv = 1.f / lsum;
-  uint16_t* os = reinterpret_cast<uint16_t*>(smem + kMerge) + hw * 32 * kKS;
+  uint16_t* os = reinterpret_cast<uint16_t*>(smem + kMerge) + wave * 32 * kKS;
 #pragma unroll
   for (int j = 0; j < kD / 32; ++j)
 #pragma unroll
@@ -374,10 +463,9 @@ __global__ __launch_bounds__(64 * W * S) void attn_fwd_kernel(FwdArgs a) {
     }
   if (hh == 0 && qrow < len)
     a.lse[static_cast<int64_t>(head) * a.n_tokens + s0 + qrow] = (m + __log2f(lsum)) * kLn2;
-  // the wavefront reads back its own staging rows (the other groups have exited: no workgroup
-  // barrier): its LDS writes complete first, and the compiler keeps the order
+  // the wavefront reads back its own staging rows: its LDS writes complete first
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  constexpr int kOut = (32 * kD / 8) / 64;  // 16-byte chunks per lane
+  constexpr int kOut = (32 * kD / 8) / 64;
   u32x4 ov[kOut];
 #pragma unroll
   for (int it = 0; it < kOut; ++it) {
@@ -385,11 +473,11 @@ __global__ __launch_bounds__(64 * W * S) void attn_fwd_kernel(FwdArgs a) {
     ov[it] = *reinterpret_cast<const u32x4*>(&os[r * kKS + 8 * cc]);
   }
   const __amdgpu_buffer_rsrc_t ors =
-      store_rsrc(a.out + static_cast<int64_t>(s0 + q0) * a.o_tok + head * a.o_head);
+      store_rsrc(a.out + static_cast<int64_t>(s0 + w0) * a.o_tok + head * a.o_head);
 #pragma unroll
   for (int it = 0; it < kOut; ++it) {
     const int cc16 = it * 64 + lane, r = cc16 / (kD / 8), cc = cc16 % (kD / 8);
-    store16(ors, q0 + r < len ? static_cast<uint32_t>((r * a.o_tok + 8 * cc) * 2) : kOob, ov[it]);
+    store16(ors, w0 + r < len ? static_cast<uint32_t>((r * a.o_tok + 8 * cc) * 2) : kOob, ov[it]);
   }
 }
 
@@ -479,27 +567,6 @@ __global__ __launch_bounds__(256) void attn_bwd_dot_kernel(BwdArgs a) {
 // loop is unrolled by two so every slot address is a compile-time offset.
 constexpr int kBwdSlot = 2 * kTileBytes + 2048;  // two tiles (+ per-wavefront lse / Dd rows: dK / dV)
 constexpr int kBwdLds = 2 * kBwdSlot;
-
-// Runs body(tile, slot) for tile = 0 .. n - 1 in ring slot tile & 1, after issue(tile + 1, slot)
-// put the next tile in flight into the other slot. Each tile's loads are waited for (this
-// wavefront's, then the barrier for everyone's) right before its body, and the barrier also
-// retires the slot the previous body read. Unrolled by two, so every slot address is a
-// compile-time offset. (A third slot, two tiles in flight, measured slower.)
-template <class Issue, class Body>
-__device__ __forceinline__ void ring2(int n, Issue&& issue, Body&& body) {
-  issue(0, 0);
-  for (int t = 0; t < n; t += 2) {
-    wait_vmcnt<0>();
-    lds_barrier();
-    if (t + 1 < n) issue(t + 1, 1);
-    body(t, 0);
-    if (t + 1 >= n) break;
-    wait_vmcnt<0>();
-    lds_barrier();
-    if (t + 2 < n) issue(t + 2, 0);
-    body(t + 1, 1);
-  }
-}
 
 // dQ: the forward's structure, one query row per lane (S^T = K Q^T, dP^T = V dO^T, then
 // dQ^T += K^T dS^T with K^T read transposed from the K tile); `tile` is the 32W-row query tile.
@@ -1001,29 +1068,42 @@ TALM_API int talm_attn_fwd(const uint16_t* q, int64_t q_stride_tok, int64_t q_st
   if (!aligned(q, 16) || !aligned(k, 16) || !aligned(v, 16) || !aligned(out, 16))
     return fail(TALM_EINVAL, "attn_fwd: q, k, v and out must be 16-byte aligned");
   const int group = n_q_heads / n_kv_heads;
-  // query heads per workgroup: the largest of 4, 3, 2, 1 that divides the group; two groups
-  // of wavefronts split each workgroup's key tiles
-  int w = 1;
-  for (int cand : {4, 3, 2})
-    if (group % cand == 0) { w = cand; break; }
+  // query heads per workgroup (4 wavefronts): 4, 2 or 1, what divides the group
+  const int h = group % 4 == 0 ? 4 : group % 2 == 0 ? 2 : 1;
+  const int rows = 32 * (4 / h);
   FwdArgs a{};
   a.q = q; a.q_tok = q_stride_tok; a.q_head = q_stride_head;
   a.k = k; a.k_tok = k_stride_tok; a.k_head = k_stride_head;
   a.v = v; a.v_tok = v_stride_tok; a.v_head = v_stride_head;
-  a.cu = cu_seqlens; a.group = group; a.head_chunks = group / w;
-  a.n_tiles = (max_seqlen + 31) / 32;
+  a.cu = cu_seqlens; a.group = group; a.head_chunks = group / h;
   a.scale_log2 = scale * 1.44269504088896341f;
   a.out = out; a.o_tok = o_stride_tok; a.o_head = o_stride_head;
   a.lse = lse; a.n_tokens = n_tokens;
-  const dim3 grid(static_cast<unsigned>(a.n_tiles), static_cast<unsigned>(n_kv_heads * a.head_chunks),
-                  static_cast<unsigned>(n_seqs));
+  // rank-major, so that every sequence's longest workgroups start first; more ranks than a grid's
+  // third axis holds go on its first one
+  const unsigned chunks = static_cast<unsigned>(n_q_heads / h), seqs = static_cast<unsigned>(n_seqs);
+  const unsigned ranks = static_cast<unsigned>((static_cast<int64_t>(max_seqlen) + rows - 1) / rows);
+  a.rank_x = ranks > 65535;
+  const dim3 grid = a.rank_x ? dim3(ranks, chunks, seqs) : dim3(chunks, seqs, ranks);
+  // Split the key tiles (S = 2) where the longest workgroup's chain, not the chip, sets the time:
+  // the workgroups (estimated: the lengths are on the device) fit one round, one per CU, and the
+  // chain is at least 8 tiles; or they fit two rounds and the chain is long enough (16 tiles) to
+  // pay for the second one. Measured, S = 1 / 2, 12 query heads on 2 KV heads: lengths [2048] 38.8 /
+  // 32.7 us, [4096] 79.7 / 66.8, [900, 700, 333] 21.0 / 18.5; [300, 211] 9.3 / 9.9; 8 rows of
+  // 128..512 15.2 / 17.7, 8 of 1024 39.4 / 47.1, [4096, 3001, 2222, 1531] 132 / 139.
+  const int64_t wgs = (n_tokens + static_cast<int64_t>(n_seqs) * rows / 2) / rows * chunks;
+  const int64_t cus = device_cus(), chain = (static_cast<int64_t>(max_seqlen) + kKeys - 1) / kKeys;
+  const bool split = wgs <= cus ? chain >= 8 : wgs <= 2 * cus && chain >= 16;
   const hipStream_t s = as_stream(stream);
-  switch (w) {
-    case 4: hipLaunchKernelGGL((attn_fwd_kernel<4, 2>), grid, dim3(512), 0, s, a); break;
-    case 3: hipLaunchKernelGGL((attn_fwd_kernel<3, 2>), grid, dim3(384), 0, s, a); break;
-    case 2: hipLaunchKernelGGL((attn_fwd_kernel<2, 2>), grid, dim3(256), 0, s, a); break;
-    default: hipLaunchKernelGGL((attn_fwd_kernel<1, 2>), grid, dim3(128), 0, s, a); break;
-  }
+#define TALM_ATTN_FWD(H)                                                                         \
+  if (split)                                                                                     \
+    hipLaunchKernelGGL((attn_fwd_kernel<H, 2>), grid, dim3(512), 0, s, a);                       \
+  else                                                                                           \
+    hipLaunchKernelGGL((attn_fwd_kernel<H, 1>), grid, dim3(256), 0, s, a)
+  if (h == 4) { TALM_ATTN_FWD(4); }
+  else if (h == 2) { TALM_ATTN_FWD(2); }
+  else { TALM_ATTN_FWD(1); }
+#undef TALM_ATTN_FWD
   return check_launch("attn_fwd");
 }
 

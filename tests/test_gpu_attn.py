@@ -43,7 +43,7 @@ def _close(name, got, ref, rel):
     assert err <= rel * scale + 1e-6, f"{name}: max error {err} > {rel} x {scale}"
 
 
-def _run(lengths, strided, seed):
+def _run(lengths, strided, seed, HQ=HQ, HKV=HKV):
     import talm_amd._ops  # noqa: F401
     from talm_amd import _ops
 
@@ -85,6 +85,20 @@ def _run(lengths, strided, seed):
 def test_attention_matches_per_row_causal_sdpa(lengths, strided, seed):
     print(f"[case] attention lengths={lengths} strided={strided} seed={seed}", flush=True)
     _run(lengths, strided, seed)
+
+
+@pytest.mark.parametrize("lengths,hq,hkv,seed", [
+    ([2048, 31], 12, 2, 11),       # few workgroups, a long chain: the key tiles split in two
+    ([449, 64, 1], 4, 1, 12),      # four heads per workgroup, split (8 key tiles), one-tile rows
+    ([448, 33], 4, 1, 13),         # the same below the split's chain length
+    ([130, 127, 128, 129], 7, 1, 14),    # one head per workgroup: 128-row tiles and their edges
+    ([320] * 24, 16, 8, 15),       # more workgroups than two rounds: unsplit, group of 2
+    ([1100, 65], 8, 8, 16),        # no grouping, split
+])
+def test_attention_over_head_groups_and_key_splits(lengths, hq, hkv, seed):
+    """Every (heads per workgroup, key split) form of the forward, at its tile edges."""
+    print(f"[case] attention lengths={lengths} heads={hq}/{hkv} seed={seed}", flush=True)
+    _run(lengths, True, seed, hq, hkv)
 
 
 def _rotate_back(dy, cos, sin):
