@@ -39,6 +39,7 @@ typedef uint16_t half4_t __attribute__((ext_vector_type(4)));
 // 16-byte register chunks as a native vector: HIP's uint4 struct is copied with memcpy, which
 // keeps a register array of them on the stack when it is stored whole into LDS.
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
 constexpr int kD = 128;         // head dim
 constexpr int kKeys = 64;       // keys per tile
@@ -134,13 +135,21 @@ __device__ __forceinline__ half8_t read16_untracked(uint32_t addr, int off) {
 }
 // Wait until at most n LDS operations are in flight (they return in order); the registers count
 // as rewritten here.
+__device__ __forceinline__ f32x4_t read_f4_untracked(uint32_t addr, int off) {
+  f32x4_t r;
+  asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(r) : "v"(addr), "n"(off));
+  return r;
+}
+// Reads that a wait for younger ones has covered already: their registers count as written here.
+__device__ __forceinline__ void lgkm_landed(f32x4_t (&r)[4]) {
+  asm volatile("" : "+v"(r[0]), "+v"(r[1]), "+v"(r[2]), "+v"(r[3]));
+}
 __device__ __forceinline__ void lgkm_wait(int n, half8_t& r) {
   asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(r) : "n"(n));
 }
 __device__ __forceinline__ void lgkm_wait(int n, half4_t& r, half4_t& q) {
   asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(r), "+v"(q) : "n"(n));
 }
-typedef float f32x4_t __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ f32x4_t read_f4_untracked(const float* lds) {
   const uint32_t addr = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
       (__attribute__((address_space(3))) const float*)(lds)));
@@ -562,11 +571,59 @@ __global__ __launch_bounds__(256) void attn_bwd_dot_kernel(BwdArgs a) {
 
 // The dQ and dK / dV bodies below stream their tiles with the forward's direct-to-LDS loads into
 // the swizzled [64][128] layout (tile_chunk): 16-byte row reads give the operands taken row by
-// row, and the transposing reads (read_tr_operand_untracked) give K^T, Q^T and dO^T straight
-// from the same tiles, so no transposed copy is written. A two-slot ring, one tile ahead; the
-// loop is unrolled by two so every slot address is a compile-time offset.
+// row, and the transposing reads give K^T, Q^T and dO^T straight from the same tiles, so no
+// transposed copy is written.
+//
+// Both walk their tiles in blocks of 32 rows, software-pipelined by hand: the products that need a
+// block's P and dS run one block behind its scores, so the exponentials of one block issue between
+// the MFMAs of another, and every operand is read from LDS into the register its last use has just
+// left, waited for with a counted lgkmcnt. The products of a tile's last block therefore still read
+// it while the next tile's scores run: a three-slot ring, one tile ahead.
+// What bounds them: one wavefront per SIMD (364 registers) issues an instruction about every 5
+// cycles, and a 64-row step of dK / dV takes 4440 cycles against 2048 of MFMAs, a 64-key step of dQ
+// 2940 against 1536 (clock stamps); taking the MFMAs out saves only 5%. Against scores,
+// exponentials and products one after the other with the operands read in batches (465
+// registers): backward of lengths [4096, 3001, 2222, 1531] 610 -> 538 us, of 16 rows of 128..512
+// 100.6 -> 94.6, of config 2's four rows 37.6 -> 35.0.
 constexpr int kBwdSlot = 2 * kTileBytes + 2048;  // two tiles (+ per-wavefront lse / Dd rows: dK / dV)
-constexpr int kBwdLds = 2 * kBwdSlot;
+constexpr int kBwdLds = 3 * kBwdSlot;
+
+// LDS addresses of a lane's operand reads: the 16-byte reads of row l32, chunks 2 s + hh, in the slot
+// the row side is at, and the transposing reads of column block j (rows 4 hh + .. and 8 rows on) in
+// the slot the transposed side is at, which follows behind. A block's rows (8 KiB), a 16-row group
+// (4 KiB) and the second tile are constant offsets.
+struct BwdReads {
+  uint32_t row[kD / 16], tlo[kD / 32], thi[kD / 32];
+  __device__ __forceinline__ void init(uint32_t lds, int lane) {
+    const int hh = lane >> 5, l32 = lane & 31, g = lane >> 4, i = lane & 15;
+#pragma unroll
+    for (int s = 0; s < kD / 16; ++s) row[s] = lds + tile_chunk(l32, 2 * s + hh) * 16;
+#pragma unroll
+    for (int j = 0; j < kD / 32; ++j) {
+      const int col = 32 * j + 16 * (g & 1) + 4 * (i & 3), r = 4 * (g >> 1) + (i >> 2);
+      tlo[j] = lds + tile_chunk(r, col >> 3) * 16 + (col & 7) * 2;
+      thi[j] = lds + tile_chunk(r + 8, col >> 3) * 16 + (col & 7) * 2;
+    }
+  }
+  __device__ __forceinline__ void next_row(uint32_t step) {
+#pragma unroll
+    for (int s = 0; s < kD / 16; ++s) row[s] += step;
+  }
+  __device__ __forceinline__ void next_t(uint32_t step) {
+#pragma unroll
+    for (int j = 0; j < kD / 32; ++j) {
+      tlo[j] += step;
+      thi[j] += step;
+    }
+  }
+};
+__device__ __forceinline__ half8_t pair8(half4_t lo, half4_t hi) {
+  return __builtin_bit_cast(half8_t, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+}
+// From one ring slot to the next, in bytes.
+__device__ __forceinline__ uint32_t slot_step(int slot) {
+  return slot == 2 ? static_cast<uint32_t>(-2 * kBwdSlot) : static_cast<uint32_t>(kBwdSlot);
+}
 
 // dQ: the forward's structure, one query row per lane (S^T = K Q^T, dP^T = V dO^T, then
 // dQ^T += K^T dS^T with K^T read transposed from the K tile); `tile` is the 32W-row query tile.
@@ -597,95 +654,139 @@ __device__ __forceinline__ void attn_bwd_dq(const BwdArgs& a, int tile, unsigned
   const float ddr = a.dd[static_cast<int64_t>(head) * a.n_tokens + s0 + qr];
   const int wq0 = q0 + 32 * wave;  // the wavefront's first query row
 
-  const int kend = min(len, q0 + kRows);
-  const int n_kt = (kend + kKeys - 1) / kKeys;
+  const int n_kt = (min(len, q0 + kRows) + kKeys - 1) / kKeys;
+  const int my_kt = (min(len, wq0 + 32) + kKeys - 1) / kKeys;  // tiles the wavefront's rows see
+  const int lim = min(qrow, len - 1) - 4 * hh;  // a lane's last key, minus its half's offset
   const uint16_t* kbase = a.k + static_cast<int64_t>(s0) * a.k_tok + kvh * a.k_head;
   const uint16_t* vbase = a.v + static_cast<int64_t>(s0) * a.v_tok + kvh * a.v_head;
-  auto issue = [&](int kt, int slot) {
+  TileDma kd, vd;
+  kd.init(a.k_tok, wave, lane);
+  vd.init(a.v_tok, wave, lane);
+  auto issue = [&](int kt, int slot) __attribute__((always_inline)) {
     unsigned char* dst = smem + slot * kBwdSlot;
     const int r0 = kt * kKeys;
-    dma_tile<W>(kbase + static_cast<int64_t>(r0) * a.k_tok, a.k_tok, len - r0, dst, wave, lane);
-    dma_tile<W>(vbase + static_cast<int64_t>(r0) * a.v_tok, a.v_tok, len - r0, dst + kTileBytes,
-                wave, lane);
+    kd.issue(kbase + static_cast<int64_t>(r0) * a.k_tok, len - r0, dst, wave);
+    vd.issue(vbase + static_cast<int64_t>(r0) * a.v_tok, len - r0, dst + kTileBytes, wave);
   };
 
-  f32x16 acc[kD / 32];
+  BwdReads rd;
+  rd.init(lds_addr(smem), lane);
+  f32x16 acc[kD / 32], st[2], dpt[2];  // block b's scores and dP in st[b], dpt[b]
 #pragma unroll
   for (int j = 0; j < kD / 32; ++j)
 #pragma unroll
     for (int v = 0; v < 16; ++v) acc[j][v] = 0.f;
-
-  auto body = [&](int kt, int slot) {
-    const unsigned char* ks = smem + slot * kBwdSlot;
-    const uint4* k16 = reinterpret_cast<const uint4*>(ks);
-    const uint4* v16 = reinterpret_cast<const uint4*>(ks + kTileBytes);
-    const int k0 = kt * kKeys;
-    if (k0 > wq0 + 31) return;  // every key of the tile is after every row of the wavefront
-    f32x16 st[2], dpt[2];
+  half8_t sb[2];     // dS^T of the block in hand, packed: 16 keys each
+  half4_t kt_[16];   // its K^T operands: [16-key group][column block][8-key halves]
+  // dS^T = P^T (dP^T - Dd), P^T = exp2(S^T scale log2e - lse2): value v of block b
+  auto value = [&](int b, int v) __attribute__((always_inline)) {
+    const float p = exp2_(__builtin_fmaf(st[b][v], a.scale_log2, -lse2));
+    sb[v >> 3][v & 7] = static_cast<_Float16>(p * (dpt[b][v] - ddr));
+  };
+  // ... 0 where masked, for the block whose first key is kb: only on a block that reaches past the
+  // wavefront's first row or past the sequence (a uniform branch that holds no MFMA: with two
+  // copies of the products the accumulators were moved between them)
+  auto mask = [&](int kb) __attribute__((always_inline)) {
+    if (kb + 31 > wq0 || kb + 32 > len) {
+      int last = lim - kb;
+      asm volatile("" : "+v"(last));  // a real branch: selects on it cannot be hoisted out
 #pragma unroll
-    for (int b = 0; b < 2; ++b) {
-#pragma unroll
-      for (int v = 0; v < 16; ++v) st[b][v] = dpt[b][v] = 0.f;
-      // the block's 16 operand reads issued before its MFMAs
-      half8_t ka[kD / 16], va[kD / 16];
-#pragma unroll
-      for (int s = 0; s < kD / 16; ++s) {
-        ka[s] = __builtin_bit_cast(half8_t, k16[tile_chunk(32 * b + l32, 2 * s + hh)]);
-        va[s] = __builtin_bit_cast(half8_t, v16[tile_chunk(32 * b + l32, 2 * s + hh)]);
-      }
-      __builtin_amdgcn_sched_group_barrier(0x100, 16, 0);
-      __builtin_amdgcn_sched_group_barrier(0x008, 16, 0);
-#pragma unroll
-      for (int s = 0; s < kD / 16; ++s) {
-        st[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ka[s], qf[s], st[b], 0, 0, 0);
-        dpt[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va[s], df[s], dpt[b], 0, 0, 0);
-      }
-    }
-    // K^T operands of the first 16-key group, read while the scores are turned into dS^T
-    half4_t kt_[2][8];
-    auto read_k = [&](int g16, int buf) {
-#pragma unroll
-      for (int j = 0; j < kD / 32; ++j)
-        read_tr_operand_untracked(ks, 16 * g16, 32 * j, lane, kt_[buf][2 * j], kt_[buf][2 * j + 1]);
-    };
-    read_k(0, 0);
-    // dS^T = P^T (dP^T - Dd), P^T = exp2(S^T scale log2e - lse2); 0 where masked (only on a tile
-    // that reaches past the wavefront's first row or past the sequence: a uniform branch)
-    if (k0 + kKeys - 1 > wq0 || k0 + kKeys > len) {
-      asm volatile("");
-#pragma unroll
-      for (int b = 0; b < 2; ++b)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const int key = k0 + 32 * b + 8 * (v >> 2) + 4 * hh + (v & 3);
-          const float p = (key <= qrow && key < len) ? exp2_(st[b][v] * a.scale_log2 - lse2) : 0.f;
-          st[b][v] = p * (dpt[b][v] - ddr);
-        }
-    } else {
-#pragma unroll
-      for (int b = 0; b < 2; ++b)
-#pragma unroll
-        for (int v = 0; v < 16; ++v)
-          st[b][v] = exp2_(st[b][v] * a.scale_log2 - lse2) * (dpt[b][v] - ddr);
-    }
-    // dQ^T[d][q] += K^T[d][key] dS^T[key][q], 16 keys per step in the accumulator's key order
-#pragma unroll
-    for (int g16 = 0; g16 < 4; ++g16) {
-      const int b = g16 >> 1, h = g16 & 1, buf = g16 & 1;
-      lgkm_wait8(kt_[buf]);
-      if (g16 < 3) read_k(g16 + 1, buf ^ 1);
-      half8_t sb;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) sb[e] = static_cast<_Float16>(st[b][8 * h + e]);
-#pragma unroll
-      for (int j = 0; j < kD / 32; ++j)
-        acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
-            __builtin_bit_cast(half8_t, __builtin_shufflevector(kt_[buf][2 * j], kt_[buf][2 * j + 1],
-                                                                0, 1, 2, 3, 4, 5, 6, 7)),
-            sb, acc[j], 0, 0, 0);
+      for (int v = 0; v < 16; ++v)
+        sb[v >> 3][v & 7] = 8 * (v >> 2) + (v & 3) <= last ? sb[v >> 3][v & 7] : static_cast<_Float16>(0.f);
     }
   };
-  ring2(n_kt, issue, body);
+  auto read_kt = [&](auto blk, int i) __attribute__((always_inline)) {  // pair i: group i / 4, block i % 4
+    constexpr int kB = decltype(blk)::value;
+    kt_[2 * i] = read_tr_untracked(rd.tlo[i & 3], kB * 8192 + (i >> 2) * 4096);
+    kt_[2 * i + 1] = read_tr_untracked(rd.thi[i & 3], kB * 8192 + (i >> 2) * 4096);
+  };
+  // block kB of the tile at the row addresses: S^T and dP^T; beside the MFMAs (kPrev) the values of
+  // the block before it, in the second half its K^T operand reads
+  auto scores = [&](auto blk, auto prev) __attribute__((always_inline)) {
+    constexpr int kB = decltype(blk)::value;
+    constexpr bool kPrev = decltype(prev)::value;
+    half8_t f[8];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      f[2 * s] = read16_untracked(rd.row[s], kB * 8192);
+      f[2 * s + 1] = read16_untracked(rd.row[s], kTileBytes + kB * 8192);
+    }
+#pragma unroll
+    for (int v = 0; v < 16; ++v) st[kB][v] = dpt[kB][v] = 0.f;
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+      const int x = 2 * (s & 3);
+      // outstanding behind the operand: the other row reads (8 while s < 4) and, from s = 5 on, 4
+      // K^T reads per step
+      lgkm_wait(s < 4 ? 7 : (7 - 2 * (s - 4)) + (kPrev ? 4 * (s - 4) : 0), f[x]);
+      st[kB] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f[x], qf[s], st[kB], 0, 0, 0);
+      if constexpr (kPrev) value(kB ^ 1, 2 * s);
+      __builtin_amdgcn_sched_barrier(0);
+      lgkm_wait(s < 4 ? 6 : (6 - 2 * (s - 4)) + (kPrev ? 4 * (s - 4) : 0), f[x + 1]);
+      dpt[kB] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f[x + 1], df[s], dpt[kB], 0, 0, 0);
+      if constexpr (kPrev) value(kB ^ 1, 2 * s + 1);
+      __builtin_amdgcn_sched_barrier(0);
+      if (s < 4) {
+        f[x] = read16_untracked(rd.row[s + 4], kB * 8192);
+        f[x + 1] = read16_untracked(rd.row[s + 4], kTileBytes + kB * 8192);
+      } else if constexpr (kPrev) {
+        read_kt(std::integral_constant<int, kB ^ 1>{}, 2 * (s - 4));
+        read_kt(std::integral_constant<int, kB ^ 1>{}, 2 * (s - 4) + 1);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  // dQ^T[d][q] += K^T[d][key] dS^T[key][q] of the block in hand, in the accumulator's key order
+  auto gather = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      lgkm_wait(14 - 2 * i, kt_[2 * i], kt_[2 * i + 1]);
+      acc[i & 3] = __builtin_amdgcn_mfma_f32_32x32x16_f16(pair8(kt_[2 * i], kt_[2 * i + 1]),
+                                                          sb[i >> 2], acc[i & 3], 0, 0, 0);
+    }
+  };
+  using B0 = std::integral_constant<int, 0>;
+  using B1 = std::integral_constant<int, 1>;
+  int slot = 0;  // of the tile in hand
+  issue(0, 0);
+  auto arrive = [&](int t) __attribute__((always_inline)) {
+    wait_vmcnt<0>();
+    lds_barrier();  // tile t has landed; everyone is done with tile t - 2, whose slot takes t + 1
+    if (t + 1 < n_kt) issue(t + 1, slot == 2 ? 0 : slot + 1);
+  };
+  auto leave = [&]() __attribute__((always_inline)) {
+    rd.next_row(slot_step(slot));
+    slot = slot == 2 ? 0 : slot + 1;
+  };
+  arrive(0);
+  scores(B0{}, std::false_type{});
+  scores(B1{}, std::true_type{});
+  mask(0);
+  gather();
+  leave();
+  for (int t = 1; t < my_kt; ++t) {
+    arrive(t);
+    scores(B0{}, std::true_type{});  // block 1 of tile t - 1: never masked, a later tile is live
+    gather();
+    rd.next_t(slot_step(slot == 0 ? 2 : slot - 1));
+    scores(B1{}, std::true_type{});
+    mask(t * kKeys);
+    gather();
+    leave();
+  }
+  // the last block: nothing to run beside it (no read is in flight here; the wait says so to a
+  // reader of the code in layout order too)
+  asm volatile("s_waitcnt lgkmcnt(0)" : "+a"(st[1]), "+a"(dpt[1]));
+#pragma unroll
+  for (int i = 0; i < 8; ++i) read_kt(B1{}, i);
+#pragma unroll
+  for (int v = 0; v < 16; ++v) value(1, v);
+  mask((my_kt - 1) * kKeys + 32);
+  gather();
+  for (int t = my_kt; t < n_kt; ++t) {  // tiles that only later rows of the workgroup see
+    arrive(t);
+    slot = slot == 2 ? 0 : slot + 1;
+  }
 
   __syncthreads();  // every wavefront is done with the ring: it becomes the output staging
   uint16_t* os = reinterpret_cast<uint16_t*>(smem) + wave * 32 * kKS;
@@ -765,6 +866,7 @@ __device__ __forceinline__ void attn_bwd_dkdv(const BwdArgs& a, int tile, unsign
   const int key = k0 + 32 * wave + l32;
   const int kr_ = min(key, len - 1);
   const int wk0 = k0 + 32 * wave;  // the wavefront's first key
+  const int q_end = key < len ? len : 0;  // a lane's query rows end here (a key past the sequence: none)
   half8_t kf[kD / 16], vf[kD / 16];
   {
     const uint16_t* kp = a.k + static_cast<int64_t>(s0 + kr_) * a.k_tok + kvh * a.k_head + 8 * hh;
@@ -783,12 +885,14 @@ __device__ __forceinline__ void attn_bwd_dkdv(const BwdArgs& a, int tile, unsign
       a.lse2 + static_cast<int64_t>(head) * a.n_tokens + s0, 0, len * 4, 0x00020000);
   const __amdgpu_buffer_rsrc_t drs = __builtin_amdgcn_make_buffer_rsrc(
       a.dd + static_cast<int64_t>(head) * a.n_tokens + s0, 0, len * 4, 0x00020000);
-  auto issue = [&](int qt, int slot) {
+  TileDma qd, od;
+  qd.init(a.q_tok, wave, lane);
+  od.init(a.do_tok, wave, lane);
+  auto issue = [&](int qt, int slot) __attribute__((always_inline)) {
     unsigned char* dst = smem + slot * kBwdSlot;
     const int r0 = qstart + qt * kRowsT;
-    dma_tile<W>(qbase + static_cast<int64_t>(r0) * a.q_tok, a.q_tok, len - r0, dst, wave, lane);
-    dma_tile<W>(dbase + static_cast<int64_t>(r0) * a.do_tok, a.do_tok, len - r0, dst + kTileBytes,
-                wave, lane);
+    qd.issue(qbase + static_cast<int64_t>(r0) * a.q_tok, len - r0, dst, wave);
+    od.issue(dbase + static_cast<int64_t>(r0) * a.do_tok, len - r0, dst + kTileBytes, wave);
     // the tile's 64 lse and 64 Dd values, one 4-byte load per lane (rows past len read 0), into
     // this wavefront's own copy (read by it alone)
     const uint32_t off = static_cast<uint32_t>((r0 + lane) * 4);
@@ -797,119 +901,156 @@ __device__ __forceinline__ void attn_bwd_dkdv(const BwdArgs& a, int tile, unsign
     __builtin_amdgcn_raw_ptr_buffer_load_lds(drs, (lds_ptr_t)(st + 256), 4, off, 0, 0, 0);
   };
 
-  f32x16 dka[kD / 32], dva[kD / 32];
+  BwdReads rd;
+  rd.init(lds_addr(smem), lane);
+  uint32_t lrow = lds_addr(smem) + 2 * kTileBytes + wave * 512 + 16 * hh;  // the rows' lse; Dd 256 on
+  f32x16 dka[kD / 32], dva[kD / 32], sc, dp;  // sc, dp: the scores and dP of the block in hand
 #pragma unroll
   for (int j = 0; j < kD / 32; ++j)
 #pragma unroll
     for (int v = 0; v < 16; ++v) dka[j][v] = dva[j][v] = 0.f;
-
-  auto body = [&](int qt, int slot) {
-    const unsigned char* qs = smem + slot * kBwdSlot;
-    const unsigned char* ds = qs + kTileBytes;
-    const uint4* q16 = reinterpret_cast<const uint4*>(qs);
-    const uint4* d16 = reinterpret_cast<const uint4*>(ds);
-    const float* ls = reinterpret_cast<const float*>(qs + 2 * kTileBytes + wave * 512);
-    const float* dds = ls + 64;
-    const int r0 = qstart + qt * kRowsT;
-    if (r0 + kRowsT - 1 < wk0) return;  // every row of the tile is before every key of the wavefront
-    // S[q][key], dP[q][key] for the tile's 32-row blocks: rows q = 32 blk + 8 (v / 4) + 4 hh + v % 4
-    f32x16 sc[2], dp[2];
+  half8_t pb[2][2], sb[2][2];  // [block][16-row group]: P and dS, packed
+  f32x4_t l4[4], d4[4];        // the block's rows' lse and Dd
+  half4_t tr[16];              // transposed operands of a 16-row group: [column block][dO, Q][halves]
+  // P and dS of value v of the block (row 8 (v / 4) + 4 hh + v % 4 of it)
+  auto value = [&](int blk, int v) __attribute__((always_inline)) {
+    const float p = exp2_(__builtin_fmaf(sc[v], a.scale_log2, -l4[v >> 2][v & 3]));
+    pb[blk][v >> 3][v & 7] = static_cast<_Float16>(p);
+    sb[blk][v >> 3][v & 7] = static_cast<_Float16>(p * (dp[v] - d4[v >> 2][v & 3]));
+  };
+  // ... 0 where masked, for the block whose first row is q0 (query row < key or past the sequence,
+  // key past the sequence): only where some row is masked for some key of the wavefront, a uniform
+  // branch that holds no MFMA (with two copies of the products the accumulators were moved)
+  auto mask = [&](int blk, int q0) __attribute__((always_inline)) {
+    if (q0 < wk0 + 31 || q0 + 32 > len || wk0 + 32 > len) {
+      int lo = key - q0 - 4 * hh;
+      const int hi = q_end - q0 - 4 * hh;
+      asm volatile("" : "+v"(lo));  // a real branch: selects on lo cannot be hoisted out of it
 #pragma unroll
-    for (int blk = 0; blk < 2; ++blk) {
-#pragma unroll
-      for (int v = 0; v < 16; ++v) sc[blk][v] = dp[blk][v] = 0.f;
-      // the block's 16 operand reads issued before its MFMAs (one LDS round trip, not one per
-      // MFMA pair)
-      half8_t qa[kD / 16], da[kD / 16];
-#pragma unroll
-      for (int s = 0; s < kD / 16; ++s) {
-        qa[s] = __builtin_bit_cast(half8_t, q16[tile_chunk(32 * blk + l32, 2 * s + hh)]);
-        da[s] = __builtin_bit_cast(half8_t, d16[tile_chunk(32 * blk + l32, 2 * s + hh)]);
-      }
-      __builtin_amdgcn_sched_group_barrier(0x100, 16, 0);  // the 16 LDS reads first
-      __builtin_amdgcn_sched_group_barrier(0x008, 16, 0);  // then the 16 MFMAs
-#pragma unroll
-      for (int s = 0; s < kD / 16; ++s) {
-        sc[blk] = __builtin_amdgcn_mfma_f32_32x32x16_f16(qa[s], kf[s], sc[blk], 0, 0, 0);
-        dp[blk] = __builtin_amdgcn_mfma_f32_32x32x16_f16(da[s], vf[s], dp[blk], 0, 0, 0);
-      }
-    }
-    // dO^T and Q^T operands of the first 16-row group, read while P and dS are formed
-    half4_t tr[2][2][8];  // [buf][dO, Q][4 j x 2 halves]
-    auto read_t = [&](int g16, int buf) {
-#pragma unroll
-      for (int j = 0; j < kD / 32; ++j) {
-        read_tr_operand_untracked(ds, 16 * g16, 32 * j, lane, tr[buf][0][2 * j], tr[buf][0][2 * j + 1]);
-        read_tr_operand_untracked(qs, 16 * g16, 32 * j, lane, tr[buf][1][2 * j], tr[buf][1][2 * j + 1]);
-      }
-    };
-    read_t(0, 0);
-    // P and dS, 0 where masked (query row < key or past the sequence, key past the sequence: only
-    // on a tile with a row before the wavefront's last key or reaching past the sequence, a
-    // uniform branch); the rows' lse and Dd come from the slot with untracked reads as well
-    const bool edge = r0 < wk0 + 31 || r0 + kRowsT > len || wk0 + 32 > len;
-#pragma unroll
-    for (int blk = 0; blk < 2; ++blk) {
-      f32x4_t l4[4], d4[4];
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        l4[g] = read_f4_untracked(&ls[32 * blk + 8 * g + 4 * hh]);
-        d4[g] = read_f4_untracked(&dds[32 * blk + 8 * g + 4 * hh]);
-      }
-      lgkm_wait_f4(l4);
-      lgkm_wait_f4(d4);
-      if (edge) {
-        asm volatile("");
-#pragma unroll
-        for (int g = 0; g < 4; ++g)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const int v = 4 * g + e, q = r0 + 32 * blk + 8 * g + 4 * hh + e;
-            const bool valid = q >= key && q < len && key < len;
-            const float p = valid ? exp2_(sc[blk][v] * a.scale_log2 - l4[g][e]) : 0.f;
-            sc[blk][v] = p;
-            dp[blk][v] = p * (dp[blk][v] - d4[g][e]);
-          }
-      } else {
-#pragma unroll
-        for (int g = 0; g < 4; ++g)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const int v = 4 * g + e;
-            const float p = exp2_(sc[blk][v] * a.scale_log2 - l4[g][e]);
-            sc[blk][v] = p;
-            dp[blk][v] = p * (dp[blk][v] - d4[g][e]);
-          }
-      }
-    }
-    // dV^T[d][key] += dO^T[d][q] P[q][key];  dK^T[d][key] += Q^T[d][q] dS[q][key]
-#pragma unroll
-    for (int g16 = 0; g16 < 4; ++g16) {
-      const int blk = g16 >> 1, h = g16 & 1, buf = g16 & 1;
-      lgkm_wait8(tr[buf][0]);
-      lgkm_wait8(tr[buf][1]);
-      if (g16 < 3) read_t(g16 + 1, buf ^ 1);
-      half8_t pb, sb;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        pb[e] = static_cast<_Float16>(sc[blk][8 * h + e]);
-        sb[e] = static_cast<_Float16>(dp[blk][8 * h + e]);
-      }
-#pragma unroll
-      for (int j = 0; j < kD / 32; ++j) {
-        dva[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
-            __builtin_bit_cast(half8_t, __builtin_shufflevector(tr[buf][0][2 * j], tr[buf][0][2 * j + 1],
-                                                                0, 1, 2, 3, 4, 5, 6, 7)),
-            pb, dva[j], 0, 0, 0);
-        dka[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
-            __builtin_bit_cast(half8_t, __builtin_shufflevector(tr[buf][1][2 * j], tr[buf][1][2 * j + 1],
-                                                                0, 1, 2, 3, 4, 5, 6, 7)),
-            sb, dka[j], 0, 0, 0);
+      for (int v = 0; v < 16; ++v) {
+        const int r = 8 * (v >> 2) + (v & 3);
+        const bool in = r >= lo && r < hi;
+        pb[blk][v >> 3][v & 7] = in ? pb[blk][v >> 3][v & 7] : static_cast<_Float16>(0.f);
+        sb[blk][v >> 3][v & 7] = in ? sb[blk][v >> 3][v & 7] : static_cast<_Float16>(0.f);
       }
     }
   };
-  ring2(n_qt, issue, body);
-
+  // operand i (column block i / 2, dO or Q) of 16-row group g of block kB
+  auto read_t = [&](auto blk, int g, int i) __attribute__((always_inline)) {
+    constexpr int kB = decltype(blk)::value;
+    const int off = kB * 8192 + g * 4096 + (i & 1 ? 0 : kTileBytes);
+    tr[2 * i] = read_tr_untracked(rd.tlo[i >> 1], off);
+    tr[2 * i + 1] = read_tr_untracked(rd.thi[i >> 1], off);
+  };
+  // block kB of the tile at the row addresses: S and dP, its lse and Dd, and (kPrev) the first group
+  // of the transposed operands of the block before it
+  auto scores = [&](auto blk, auto prev) __attribute__((always_inline)) {
+    constexpr int kB = decltype(blk)::value;
+    constexpr bool kPrev = decltype(prev)::value;
+    half8_t f[8];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      f[2 * s] = read16_untracked(rd.row[s], kB * 8192);
+      f[2 * s + 1] = read16_untracked(rd.row[s], kTileBytes + kB * 8192);
+    }
+#pragma unroll
+    for (int g = 0; g < 4; ++g) l4[g] = read_f4_untracked(lrow, kB * 128 + g * 32);
+#pragma unroll
+    for (int g = 0; g < 4; ++g) d4[g] = read_f4_untracked(lrow, 256 + kB * 128 + g * 32);
+#pragma unroll
+    for (int v = 0; v < 16; ++v) sc[v] = dp[v] = 0.f;
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+      const int x = 2 * (s & 3);
+      // outstanding behind the operand: s < 4: the other row reads and the 8 lse / Dd reads, 15;
+      // then the other row reads and, from s = 5 on, 4 transposed reads per step
+      lgkm_wait(s < 4 ? 15 : (7 - 2 * (s - 4)) + (kPrev ? 4 * (s - 4) : 0), f[x]);
+      sc = __builtin_amdgcn_mfma_f32_32x32x16_f16(f[x], kf[s], sc, 0, 0, 0);
+      lgkm_wait(s < 4 ? 14 : (6 - 2 * (s - 4)) + (kPrev ? 4 * (s - 4) : 0), f[x + 1]);
+      dp = __builtin_amdgcn_mfma_f32_32x32x16_f16(f[x + 1], vf[s], dp, 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      if (s < 4) {
+        f[x] = read16_untracked(rd.row[s + 4], kB * 8192);
+        f[x + 1] = read16_untracked(rd.row[s + 4], kTileBytes + kB * 8192);
+      } else if constexpr (kPrev) {
+        read_t(std::integral_constant<int, kB ^ 1>{}, 0, 2 * (s - 4));
+        read_t(std::integral_constant<int, kB ^ 1>{}, 0, 2 * (s - 4) + 1);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    // the lse / Dd reads have returned (they were issued before the second row reads)
+    lgkm_landed(l4);
+    lgkm_landed(d4);
+  };
+  // dV^T[d][key] += dO^T[d][q] P[q][key], dK^T[d][key] += Q^T[d][q] dS[q][key] of block kB (its first
+  // group's operands in flight); beside each MFMA (kNext) a value of the other block
+  auto gather = [&](auto blk, auto next) __attribute__((always_inline)) {
+    constexpr int kB = decltype(blk)::value;
+    constexpr bool kNext = decltype(next)::value;
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+      const int g = u >> 3, i = u & 7, j = i >> 1;
+      lgkm_wait(g == 0 ? 14 : 14 - 2 * i, tr[2 * i], tr[2 * i + 1]);
+      if (i & 1)
+        dka[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(pair8(tr[2 * i], tr[2 * i + 1]), sb[kB][g], dka[j], 0, 0, 0);
+      else
+        dva[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(pair8(tr[2 * i], tr[2 * i + 1]), pb[kB][g], dva[j], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      if (g == 0) read_t(blk, 1, i);
+      if constexpr (kNext) value(kB ^ 1, u);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  using B0 = std::integral_constant<int, 0>;
+  using B1 = std::integral_constant<int, 1>;
+  const int t0 = (wk0 - qstart) / kRowsT;  // the first tile with a row at or past the wavefront's keys
+  int slot = 0;  // of the tile in hand
+  issue(0, 0);
+  auto arrive = [&](int t) __attribute__((always_inline)) {
+    wait_vmcnt<0>();
+    lds_barrier();  // tile t has landed; everyone is done with tile t - 2, whose slot takes t + 1
+    if (t + 1 < n_qt) issue(t + 1, slot == 2 ? 0 : slot + 1);
+  };
+  auto leave = [&]() __attribute__((always_inline)) {
+    rd.next_row(slot_step(slot));
+    lrow += slot_step(slot);
+    slot = slot == 2 ? 0 : slot + 1;
+  };
+  for (int t = 0; t < t0 && t < n_qt; ++t) {
+    arrive(t);
+    rd.next_t(slot_step(slot));
+    leave();
+  }
+  if (t0 < n_qt) {
+    const int q0 = qstart + t0 * kRowsT;
+    arrive(t0);
+    scores(B0{}, std::false_type{});
+#pragma unroll
+    for (int v = 0; v < 16; ++v) value(0, v);
+    mask(0, q0);
+    scores(B1{}, std::true_type{});
+    gather(B0{}, std::true_type{});
+    mask(1, q0 + 32);
+    leave();
+    for (int t = t0 + 1; t < n_qt; ++t) {
+      const int r0 = qstart + t * kRowsT;
+      arrive(t);
+      scores(B0{}, std::true_type{});
+      gather(B1{}, std::true_type{});
+      mask(0, r0);
+      rd.next_t(slot_step(slot == 0 ? 2 : slot - 1));
+      scores(B1{}, std::true_type{});
+      gather(B0{}, std::true_type{});
+      mask(1, r0 + 32);
+      leave();
+    }
+    // the last block: nothing to run beside it (as in dQ: no read is in flight)
+    asm volatile("s_waitcnt lgkmcnt(0)");
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) read_t(B1{}, 0, i);
+    gather(B1{}, std::false_type{});
+  }
   // fp32 partials [head][token][d]. A lane holds its key's column of the accumulators (rows
   // d = 32 j + 8 (v / 4) + 4 hh + v % 4): stored as they are, every store instruction would touch
   // 64 rows 16 bytes each. Each wavefront stages its 32 keys x 128 columns in its own part of the
