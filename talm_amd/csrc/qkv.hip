@@ -155,8 +155,11 @@ __global__ __launch_bounds__(64 * kDownWaves) void lora_down_kernel(
 // the token count gives few row tiles, so the smaller tile doubles the workgroups in flight and
 // each keeps its own L2 -> LDS stream busy.
 using QkvShape = TileShape<64, 128, 64, 3, 2, 2>;
+// Where that gives more than one round of workgroups, 128 x 128 tiles of 64 x 64 per wavefront: a
+// third fewer operand bytes from L2 and LDS per product, in a two-slot ring (64 KiB) so that two
+// still share a CU.
+using QkvWide = TileShape<128, 128, 64, 2, 2, 2>;
 constexpr int kQZS = QkvShape::kBN + 8;             // staged tile row stride (halfs)
-static_assert(QkvShape::kBM * kQZS * 2 <= QkvShape::kRing, "the staged tile reuses the ring");
 
 // An operand whose k range has two parts: steps [0, nk1) read `base1` (k < k1), the steps after
 // them read `base2` (k in [lo2, hi2), counted from 0 again). The per-lane row and chunk do not depend on the part; the
@@ -225,6 +228,7 @@ struct QkvArgs {
   const float* sin;
   int64_t cs_stride;
   int rope_cols;          // columns [0, rope_cols) are heads of 128 to rotate
+  int cs_vec;             // cos / sin rows are 16-byte aligned
   uint16_t* out;          // [n_tokens][ldo]
   int64_t ldo;
   int n_mtiles, n_ntiles;
@@ -251,16 +255,17 @@ constexpr int kDownSlice = kRank * 64 * 2;  // bytes of one step's A_g slice
 template <class S>
 struct DownHook {
   static constexpr int kLoads = 1;
+  static constexpr int kBlocks = S::kBM / 64;  // 16-row blocks per wavefront
   __amdgpu_buffer_rsrc_t ra;
   unsigned char* ring;  // kStages slices of kDownSlice bytes
   uint32_t off;         // this lane's global byte offset at step 0 (lanes below 32)
   int klim;             // k below which A_g is read: the hidden size, 0 outside the adapters
   int kc;               // this lane's k inside a step (lanes below 32)
   int dst;              // this wavefront's 512 bytes of a slice
-  int row;              // the lane's x row in the stage: 16 wave + lane % 16
+  int row;              // the lane's x row in the stage: 16 kBlocks wave + lane % 16 (+ 16 per block)
   int lane;
   bool live;            // the tile is in an adapter's columns
-  f32x4 t;
+  f32x4 t[kBlocks];
   __device__ __forceinline__ void prefetch(int kt, int slot) {
     const int k = kt * S::kBK + kc;
     // one compare, no branch around the address: a select between two offsets
@@ -276,9 +281,11 @@ struct DownHook {
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       const int c = 4 * h + (lane >> 4);
-      t = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, As[swz<S::kCpr>(row, c)]),
-                                                  __builtin_bit_cast(half8_t, Bs[r * 8 + (c ^ (r >> 1))]),
-                                                  t, 0, 0, 0);
+      const half8_t b = __builtin_bit_cast(half8_t, Bs[r * 8 + (c ^ (r >> 1))]);
+#pragma unroll
+      for (int i = 0; i < kBlocks; ++i)
+        t[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+            __builtin_bit_cast(half8_t, As[swz<S::kCpr>(row + 16 * i, c)]), b, t[i], 0, 0, 0);
     }
   }
 };
@@ -288,17 +295,26 @@ struct DownHook {
 // kDown: the forward with the adapters' t = x A_g^T computed by the tile itself during the main
 // product (DownHook) and the adapter term added after it as ts B_g^T (ts = fp16(scaling t),
 // two v_mfma_f32_32x32x16_f16 per wavefront, K = the rank 16), in place of the extra step.
-constexpr int kTsOff = 32 * 1024;  // ts [64][kTsLd] in the ring after the main product
-constexpr int kTsLd = 24;          // 48-byte rows: a 16-lane phase of 16-byte reads meets 16 bank groups
-static_assert(kTsOff >= QkvShape::kBM * kQZS * 2 && kTsOff + QkvShape::kBM * kTsLd * 2 <= QkvShape::kRing,
-              "ts beside the staged tile");
+constexpr int kTsLd = 24;  // 48-byte rows: a 16-lane phase of 16-byte reads meets 16 bank groups
 
-template <bool kDown>
-__global__ __launch_bounds__(QkvShape::kThreads, QkvShape::kPerCu) void proj_ext_kernel(QkvArgs a) {
-  using S = QkvShape;
-  static_assert(S::kFragM == 1 && S::kWaveM == 32 && S::kWaves == 4 && S::kBM == 64 &&
-                    S::kBK == 64 && S::kCpr == 8,
-                "the down-projection hook assumes four wavefronts on 64 rows, 64-deep steps");
+// Eight consecutive floats; `vec`: 16-byte aligned.
+__device__ __forceinline__ void load8f(const float* p, bool vec, float (&v)[8]) {
+  if (vec) {
+    const float4 a = reinterpret_cast<const float4*>(p)[0], b = reinterpret_cast<const float4*>(p)[1];
+    v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
+    v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+  } else {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = p[e];
+  }
+}
+
+template <class S, bool kDown>
+__global__ __launch_bounds__(S::kThreads, S::kPerCu) void proj_ext_kernel(QkvArgs a) {
+  static_assert(S::kWaves == 4 && S::kBM % 64 == 0 && S::kBN == 128 && S::kBK == 64 && S::kCpr == 8,
+                "four wavefronts, 64-deep steps, whole heads per tile");
+  constexpr int kTsOff = (S::kBM * kQZS * 2 + 1023) / 1024 * 1024;  // ts [kBM][kTsLd] behind the staged tile
+  static_assert(kTsOff + S::kBM * kTsLd * 2 <= S::kRing, "the staged tile and ts reuse the ring");
   // the tile ring, then (kDown) the adapter slices' ring
   __shared__ __attribute__((aligned(1024))) unsigned char smem[S::kRing + (kDown ? S::kStages * kDownSlice : 0)];
   const uint32_t tile = xcd_tile(blockIdx.x, static_cast<uint32_t>(a.n_mtiles * a.n_ntiles));
@@ -362,9 +378,10 @@ __global__ __launch_bounds__(QkvShape::kThreads, QkvShape::kPerCu) void proj_ext
     hook.dst = wave * 512;
     hook.lane = lane;
     hook.klim = g >= 0 ? a.hidden : 0;
-    hook.row = 16 * wave + (lane & 15);
+    hook.row = 16 * DownHook<S>::kBlocks * wave + (lane & 15);
     hook.live = g >= 0;
-    hook.t = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < DownHook<S>::kBlocks; ++i) hook.t[i] = f32x4{0.f, 0.f, 0.f, 0.f};
     ring_gemm<S>(
         smem, nk1,
         [&](unsigned char* slot, int kt) {
@@ -378,19 +395,25 @@ __global__ __launch_bounds__(QkvShape::kThreads, QkvShape::kPerCu) void proj_ext
     if (g >= 0) {
       const float sg = g1 ? a.scaling[1] : a.scaling[0];
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int r = 16 * wave + 4 * (lane >> 4) + v;
-        tsl[r * kTsLd + (lane & 15)] = f2h(sg * hook.t[v]);
-        if (n0 == sb && m0 + r < a.n_tokens)
-          a.t_out[static_cast<int64_t>(m0 + r) * a.ldt_out + kRank * g + (lane & 15)] = f2h(hook.t[v]);
-      }
+      for (int i = 0; i < DownHook<S>::kBlocks; ++i)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int r = 16 * (DownHook<S>::kBlocks * wave + i) + 4 * (lane >> 4) + v;
+          tsl[r * kTsLd + (lane & 15)] = f2h(sg * hook.t[i][v]);
+          if (n0 == sb && m0 + r < a.n_tokens)
+            a.t_out[static_cast<int64_t>(m0 + r) * a.ldt_out + kRank * g + (lane & 15)] = f2h(hook.t[i][v]);
+        }
     }
     __syncthreads();  // every wavefront's ts rows are in LDS
     if (g >= 0) {
-      const half8_t tsa = *reinterpret_cast<const half8_t*>(&tsl[(wm * S::kWaveM + (lane & 31)) * kTsLd + 8 * (lane >> 5)]);
 #pragma unroll
-      for (int j = 0; j < S::kFragN; ++j)
-        acc[0][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(tsa, bfr[j], acc[0][j], 0, 0, 0);
+      for (int i = 0; i < S::kFragM; ++i) {
+        const half8_t tsa = *reinterpret_cast<const half8_t*>(
+            &tsl[(wm * S::kWaveM + 32 * i + (lane & 31)) * kTsLd + 8 * (lane >> 5)]);
+#pragma unroll
+        for (int j = 0; j < S::kFragN; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(tsa, bfr[j], acc[i][j], 0, 0, 0);
+      }
     }
   }
 
@@ -406,26 +429,31 @@ __global__ __launch_bounds__(QkvShape::kThreads, QkvShape::kPerCu) void proj_ext
       for (int v = 0; v < 16; ++v) Zs[acc_row<S>(wm, i, v, lane) * kQZS + col] = f2h(acc[i][j][v] + bv);
     }
   __syncthreads();
-  if (a.cos && n0 < a.rope_cols) {
-    // one head: y1 = x1 c1 - x2 s1, y2 = x2 c2 + x1 s2 on the pairs (j, j + 64)
-    for (int e = tid; e < S::kBM * 64; e += S::kThreads) {
-      const int row = e >> 6, j = e & 63, gr = m0 + row;
-      if (gr >= a.n_tokens) continue;
-      const float* cr = a.cos + static_cast<int64_t>(gr) * a.cs_stride;
-      const float* sr = a.sin + static_cast<int64_t>(gr) * a.cs_stride;
-      const float x1 = h2f(Zs[row * kQZS + j]), x2 = h2f(Zs[row * kQZS + j + 64]);
-      Zs[row * kQZS + j] = f2h(x1 * cr[j] - x2 * sr[j]);
-      Zs[row * kQZS + j + 64] = f2h(x2 * cr[j + 64] + x1 * sr[j + 64]);
-    }
-    __syncthreads();
-  }
-#pragma unroll
+  // 16-byte row stores; on a rotated head, y1 = x1 c1 - x2 s1, y2 = x2 c2 + x1 s2 on the pairs
+  // (j, j + 64): a thread's eight columns with their eight partners, read beside them. (Element by
+  // element in LDS with a barrier before the stores, the rotation cost 20 us at 5015 tokens.)
+  const bool rot = a.cos && n0 < a.rope_cols;
+#pragma unroll 4
   for (int it = 0; it < (S::kBM * S::kBN / 8) / S::kThreads; ++it) {
     const int c = it * S::kThreads + tid, row = c >> 4, kc = c & 15;
     const int gr = m0 + row, gc = n0 + kc * 8;
-    if (gr < a.n_tokens && gc < a.n_out)
-      *reinterpret_cast<uint4*>(a.out + static_cast<int64_t>(gr) * a.ldo + gc) =
-          *reinterpret_cast<const uint4*>(Zs + row * kQZS + kc * 8);
+    if (gr >= a.n_tokens || gc >= a.n_out) continue;
+    uint4 z = *reinterpret_cast<const uint4*>(Zs + row * kQZS + kc * 8);
+    if (rot) {
+      const uint4 p = *reinterpret_cast<const uint4*>(Zs + row * kQZS + (kc ^ 8) * 8);
+      float cv[8], sv[8];
+      load8f(a.cos + static_cast<int64_t>(gr) * a.cs_stride + kc * 8, a.cs_vec, cv);
+      load8f(a.sin + static_cast<int64_t>(gr) * a.cs_stride + kc * 8, a.cs_vec, sv);
+      const uint32_t zw[4] = {z.x, z.y, z.z, z.w}, pw[4] = {p.x, p.y, p.z, p.w};
+      const float sign = kc < 8 ? -1.f : 1.f;
+      uint32_t y[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        y[e] = pack2(lo_f(zw[e]) * cv[2 * e] + sign * lo_f(pw[e]) * sv[2 * e],
+                     hi_f(zw[e]) * cv[2 * e + 1] + sign * hi_f(pw[e]) * sv[2 * e + 1]);
+      z = make_uint4(y[0], y[1], y[2], y[3]);
+    }
+    *reinterpret_cast<uint4*>(a.out + static_cast<int64_t>(gr) * a.ldo + gc) = z;
   }
 }
 
@@ -764,20 +792,26 @@ int check_proj(const char* what, int64_t ldx, int64_t n_tokens, int64_t hidden, 
   return TALM_OK;
 }
 
-void launch_proj(QkvArgs& a, hipStream_t stream) {
-  using S = QkvShape;
+template <class S, bool kDown>
+void launch_tiles(QkvArgs& a, hipStream_t stream) {
   a.n_mtiles = (a.n_tokens + S::kBM - 1) / S::kBM;
   a.n_ntiles = (a.n_out + S::kBN - 1) / S::kBN;
-  hipLaunchKernelGGL(proj_ext_kernel<false>, dim3(static_cast<unsigned>(a.n_mtiles * a.n_ntiles)),
+  hipLaunchKernelGGL((proj_ext_kernel<S, kDown>), dim3(static_cast<unsigned>(a.n_mtiles * a.n_ntiles)),
                      dim3(S::kThreads), 0, stream, a);
 }
 
-void launch_proj_down(QkvArgs& a, hipStream_t stream) {
-  using S = QkvShape;
-  a.n_mtiles = (a.n_tokens + S::kBM - 1) / S::kBM;
-  a.n_ntiles = (a.n_out + S::kBN - 1) / S::kBN;
-  hipLaunchKernelGGL(proj_ext_kernel<true>, dim3(static_cast<unsigned>(a.n_mtiles * a.n_ntiles)),
-                     dim3(S::kThreads), 0, stream, a);
+template <bool kDown>
+void launch_proj(QkvArgs& a, hipStream_t stream) {
+  a.cs_vec = a.cos && aligned(a.cos, 16) && aligned(a.sin, 16) && a.cs_stride % 4 == 0;
+  // 128-row tiles once the 64-row ones exceed one round at two workgroups per CU. Measured, 64 / 128
+  // rows: forward at 3000 tokens 46.5 / 36.6 us, at 5015 73.0 / 68.8, input gradient 41.3 / 31.9 and 54.7 /
+  // 39.2; at 2048 tokens and below (one round of 64-row tiles) half as many workgroups would run.
+  const int64_t small = static_cast<int64_t>((a.n_tokens + QkvShape::kBM - 1) / QkvShape::kBM) *
+                        ((a.n_out + QkvShape::kBN - 1) / QkvShape::kBN);
+  if (small > 2 * device_cus() && fits32(QkvWide::kBM, a.ldx))
+    launch_tiles<QkvWide, kDown>(a, stream);
+  else
+    launch_tiles<QkvShape, kDown>(a, stream);
 }
 
 }  // namespace
@@ -831,7 +865,7 @@ TALM_API int talm_qkv_lora_fwd(const uint16_t* x, int64_t ldx, int64_t n_tokens,
   }
   a.cos = cos; a.sin = sin; a.cs_stride = cs_stride; a.rope_cols = static_cast<int>(rope_cols);
   a.out = out; a.ldo = ldo;
-  launch_proj(a, as_stream(stream));
+  launch_proj<false>(a, as_stream(stream));
   return check_launch("qkv_lora_fwd");
 }
 
@@ -889,7 +923,7 @@ TALM_API int talm_qkv_lora_fwd_down(const uint16_t* x, int64_t ldx, int64_t n_to
   a.t_out = t; a.ldt_out = ldt;
   a.cos = cos; a.sin = sin; a.cs_stride = cs_stride; a.rope_cols = static_cast<int>(rope_cols);
   a.out = out; a.ldo = ldo;
-  launch_proj_down(a, as_stream(stream));
+  launch_proj<true>(a, as_stream(stream));
   return check_launch("qkv_lora_fwd_down");
 }
 
@@ -948,7 +982,7 @@ TALM_API int talm_qkv_lora_bwd_dx(const uint16_t* dcat, int64_t ldc, int64_t n_t
   a.seg_begin[0] = 0; a.seg_end[0] = static_cast<int>(hidden);
   a.k_lo[0] = 0; a.k_hi[0] = static_cast<int>(rank);
   a.out = dx; a.ldo = lddx;
-  launch_proj(a, as_stream(stream));
+  launch_proj<false>(a, as_stream(stream));
   return check_launch("qkv_lora_bwd_dx");
 }
 

@@ -163,6 +163,33 @@ def test_qkv_lora_fwd_down_matches_fp32(n, size, n_out, segs, rope_cols, with_bi
         assert torch.all((out.float() - out2.float()).abs() <= 2e-3 * out2.float().abs() + 1e-3 * scale)
 
 
+@pytest.mark.parametrize("n", [2113, 2176])  # 128-row tiles: a last tile of 65 rows, a full one
+def test_projections_on_128_row_tiles(n):
+    """More than one round of 64-row tiles: the 128-row kernels, forward with the adapters'
+    down-projection, forward from ts, and the input gradient, against the same references."""
+    segs = [(0, 1536), (1792, 2048)]
+    test_qkv_lora_fwd_down_matches_fp32(n, 192, 2048, segs, 1792, True)
+    test_qkv_lora_fwd_matches_fp32(n, 192, 2048, segs, 1792, True)
+    test_qkv_lora_bwd_dx_matches_fp32(n, 2048, 256, 32)
+
+
+def test_rotation_with_unaligned_tables():
+    """cos / sin rows that are not 16-byte aligned (row stride 129) rotate to the same bits."""
+    n, size, n_out = 77, 64, 384
+    x, w, bias, _a, _b = _inputs(n, size, n_out, [], seed=5)
+    cos, sin = _rope_tables(n)
+    outs = []
+    for stride in (128, 129):
+        tables = [torch.zeros(n, stride, device=DEV) for _ in range(2)]
+        for t, src in zip(tables, (cos, sin)):
+            t[:, :128] = src
+        out = torch.empty(n, n_out, dtype=torch.float16, device=DEV)
+        torch.ops.talm.qkv_lora_fwd(x, w, bias, None, None, 0, 0, None, 0, 0, tables[0], tables[1],
+                                    256, out)
+        outs.append(out)
+    assert torch.equal(*outs)
+
+
 def test_qkv_lora_fwd_rejects_misaligned_adapter_columns():
     _case("qkv_lora_fwd rejects")
     x, w, bias, a, b = _inputs(8, 64, 512, [(64, 192)], seed=1)
