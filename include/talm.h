@@ -217,9 +217,11 @@ int talm_swiglu_bwd_rows(const uint16_t* grad, int64_t ld_grad, const uint16_t* 
                          int64_t cols, void* stream);
 
 /*
- * Bytes of workspace talm_head_ce needs (-1 for arguments it would reject). `group` vocabulary
- * slices are processed per step: the workspace holds their fp16 logits [n_rows, group * vchunk],
- * the per-tile statistics and the fp32 gradient partials [group, n_grad, hidden].
+ * Bytes of workspace talm_head_ce needs (-1 for arguments it would reject). At least
+ * `group` vocabulary slices are processed per step, more where few rows leave room (the gradient
+ * rows' e^{z - m} within 168 MiB; without gradient rows, the statistics within 64 MiB): the workspace
+ * holds a step's fp16 e^{z - m} [n_grad, slices * vchunk], its per-tile statistics and the fp32
+ * gradient partials [parts, n_grad, hidden].
  */
 int64_t talm_head_ce_workspace(int64_t n_rows, int64_t hidden, int64_t vocab, int64_t vchunk,
                                int64_t n_grad, int32_t group);
@@ -234,7 +236,8 @@ int talm_head_weight_t(const uint16_t* weight, int64_t ldw, int64_t vocab, int64
 
 /*
  * Fused LM head + cross-entropy over the vocabulary in slices of `vchunk` columns (a multiple of
- * 128), forward and gradient in one call; the [n_rows, vocab] logits never exist.
+ * 128), forward and gradient in one call; no [n_rows, vocab] logits (of a step's columns, the
+ * gradient rows' e^{z - m} in fp16).
  * Replaces FusedHeadLossVocab.forward's slice loop with torch.mm, launch_vocab /
  * fused_head_vocab_kernel and the accumulator addmm (solution/fused_head.py:88-182, :236-251,
  * :356-383).
@@ -250,7 +253,8 @@ int talm_head_weight_t(const uint16_t* weight, int64_t ldw, int64_t vocab, int64
  * best_idx == target); and, when grad_hidden is not NULL, grad_hidden f16 [n_rows, hidden]
  * (row stride hidden): dH = acc / s - W[target] for labelled rows, 0 for the others, with
  * acc = sum over slices of the reference's rescaled fp16(e^{z - m}) W products.
- * `workspace` (256-byte aligned) holds talm_head_ce_workspace(...) bytes.
+ * `workspace` (256-byte aligned) holds talm_head_ce_workspace(...) bytes; one that holds only a
+ * step of `group` slices is accepted too (the loop then takes `group` at a time).
  */
 int talm_head_ce(const uint16_t* hidden_states, int64_t ldh, const uint16_t* weight, int64_t ldw,
                  const int64_t* targets, int64_t n_rows,

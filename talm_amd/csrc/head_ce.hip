@@ -6,7 +6,8 @@
 // and for labelled rows the gradient accumulator: acc = e^{m_old - m} acc + fp16(e^{z-m}) W_c,
 // with m the running maximum after slice c; at the end dH = acc / s - W[target].
 //
-// The same recurrence here, shaped for MI355X. Slices are processed `group` at a time:
+// The same recurrence here, shaped for MI355X. Slices are processed a group at a time (`group` of
+// them or, with few rows, more: slices_per_step):
 //   head_logits   Z = H W^T over the group's columns; the epilogue rounds to fp16, stages the
 //                 tile in LDS and emits, per (row, 128-column tile), the tile's max m_t, first
 //                 argmax, sum e^{z-m_t} and sum e^{z-m_t} z; for labelled rows it also writes
@@ -25,7 +26,7 @@
 //                 accumulator update up to one more fp16 rounding of P.
 //   head_combine  acc = e^{m_prev - m_G} acc + the parts' sum, and after the last group
 //                 dH = acc / s - W16[target] in fp16.
-// The full [N, V] logits never exist: one group of slices (group * vchunk columns) at a time.
+// The full [N, V] logits never exist, only P for the gradient rows and one group's columns.
 //
 // Both GEMMs run the tile core of mfma_tile.h (v_mfma_f32_32x32x16_f16, operands streamed by
 // buffer_load_dwordx4 ... lds straight into an LDS ring, 16-byte chunks XOR-swizzled so that
@@ -36,6 +37,7 @@
 #include "mfma_tile.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace talm {
 namespace {
@@ -328,8 +330,18 @@ __global__ __launch_bounds__(S::kThreads, 1) void head_logits_kernel(LogitsArgs 
   Loader<S, S::kBN> lb;
   la.lanes(a.ldw, a.K, wave, lane);
   lb.lanes(a.ldh, a.K, wave, lane);
+  // Token tiles vary fastest. Where the stride is a multiple of their number, a workgroup would meet
+  // the same token tile every time, and the last, partly empty one costs less: the tokens are
+  // rotated by one every `stride` tiles (by the vocabulary tile, so the map stays one to one).
+  const uint32_t n_tt = static_cast<uint32_t>(a.n_ttiles), turn = max(stride / n_tt, 1u);
+  auto tile_of = [&](uint32_t tile, int& tt, int& vt) {
+    const uint32_t v = tile / n_tt;
+    vt = static_cast<int>(v);
+    tt = static_cast<int>((tile - v * n_tt + v / turn) % n_tt);
+  };
   auto start_tile = [&](uint32_t tile) {
-    const int tt = static_cast<int>(tile % a.n_ttiles), vt = static_cast<int>(tile / a.n_ttiles);
+    int tt, vt;
+    tile_of(tile, tt, vt);
     la.rows(a.W + static_cast<int64_t>(vt) * S::kBM * a.ldw, a.ldw, min(a.group_cols - vt * S::kBM, S::kBM));
     lb.rows(a.H + static_cast<int64_t>(tt) * S::kBN * a.ldh, a.ldh, min(a.n_rows - tt * S::kBN, S::kBN));
     if (nk > 0) {
@@ -344,7 +356,11 @@ __global__ __launch_bounds__(S::kThreads, 1) void head_logits_kernel(LogitsArgs 
   if (first >= end) return;
   start_tile(first);
   for (uint32_t tile = first;;) {
-    const int tt = static_cast<int>(tile % a.n_ttiles), vt = static_cast<int>(tile / a.n_ttiles);
+    int tt, vt;
+    tile_of(tile, tt, vt);
+    // a wavefront whose 64 tokens all lie past the last row (in the last token tile) has nothing
+    // to compute; it keeps its share of the loads and the barriers
+    const bool live = tt * S::kBN + wn * S::kWaveN < a.n_rows;
     const int c0 = vt * S::kBM + wm * S::kWaveM;  // the wavefront's first column in the group
     const int valid = a.group_cols - c0;         // of its rows, those that are vocabulary
     // the targets of the lane's two tokens, loaded before the K loop (whose first wait covers
@@ -385,21 +401,26 @@ __global__ __launch_bounds__(S::kThreads, 1) void head_logits_kernel(LogitsArgs 
             acc[i][j][v] =
                 __int_as_float(((lim - (i * 32 + 8 * (v >> 2) + (v & 3))) >> 31) & kLowest);
     }
-    for (int kb = 0; kb < nk; kb += kSt) {
+    auto k_loop = [&](auto compute) __attribute__((always_inline)) {
+      for (int kb = 0; kb < nk; kb += kSt) {
 #pragma unroll
-      for (int i = 0; i < kSt; ++i) {  // step kt = kb + i in slot i
-        const int kt = kb + i;
-        if (kt >= nk) break;
-        wait_vmcnt<0>();  // this step's group (and, at step 0, the previous epilogue's stores)
-        lds_barrier();
-        if (kt + 1 < nk) {
-          unsigned char* slot = smem + ((i + 1) % kSt) * S::kStageBytes;
-          la.issue(slot, (kt + 1) * S::kBK, wave);
-          lb.issue(slot + S::kAChunks * 16, (kt + 1) * S::kBK, wave);
+        for (int i = 0; i < kSt; ++i) {  // step kt = kb + i in slot i
+          const int kt = kb + i;
+          if (kt >= nk) break;
+          wait_vmcnt<0>();  // this step's group (and, at step 0, the previous epilogue's stores)
+          lds_barrier();
+          if (kt + 1 < nk) {
+            unsigned char* slot = smem + ((i + 1) % kSt) * S::kStageBytes;
+            la.issue(slot, (kt + 1) * S::kBK, wave);
+            lb.issue(slot + S::kAChunks * 16, (kt + 1) * S::kBK, wave);
+          }
+          if constexpr (compute.value) logits_step<S>(smem + i * S::kStageBytes, fo, acc);
         }
-        logits_step<S>(smem + i * S::kStageBytes, fo, acc);
       }
-    }
+    };
+    // two loops rather than a branch in the step: the branch cost every full tile 1.2%
+    if (live) k_loop(std::true_type{});
+    else k_loop(std::false_type{});
     // the targets count as written here, where nothing else is in flight: their wait (if the
     // loop's own did not cover them) is placed here and not after the next step's loads below
     asm volatile("" : "+v"(tgt[0]), "+v"(tgt[1]));
@@ -428,7 +449,7 @@ __global__ __launch_bounds__(S::kThreads, 1) void head_logits_kernel(LogitsArgs 
       mx[j] = fmaxf(static_cast<float>(m2[0]), static_cast<float>(m2[1]));
     }
     uint16_t* zs = reinterpret_cast<uint16_t*>(smem + S::kStageBytes) + tid * 64;
-    if (valid > 0) {
+    if (valid > 0 && live) {
 #pragma unroll
       for (int j = 0; j < S::kFragN; ++j) {
         const int tok = tt * S::kBN + wn * S::kWaveN + j * 32 + (lane & 31);
@@ -461,8 +482,8 @@ struct MergeArgs {
   int n_rows;
   int n_grad;
   int n_slices;            // slices in this group
-  int slice_cols[8];       // columns of each slice (the last may be narrower)
-  int slice_col0[8];       // first vocabulary column of each slice
+  int col0;                // the group's first vocabulary column
+  int vocab;
   int vchunk;              // columns per full slice (a multiple of kTile)
   int first_slice;         // this group holds the first slice of the vocabulary
   int last_slice;          // this group holds the last slice
@@ -474,25 +495,29 @@ struct MergeArgs {
   int32_t* correct;
 };
 
+constexpr int kSliceLoads = 8;  // slices whose tiles a lane of head_merge holds at a time
+
 // One wavefront per row. With slices of at most 64 tiles (vchunk <= 8192) a lane holds one tile of
 // each slice, and every load the row needs (the group's tiles, the running statistics, the
 // target's logit) is issued before the first reduction: one memory round trip per row instead
-// of two per slice. Wider slices take the tiles in lane-strided loops. Same merges in the same
-// order either way.
+// of two per slice (of a group of more than eight slices, eight at a time). Wider slices take the
+// tiles in lane-strided loops. Same merges in the same order either way.
 template <bool kOne>
 __device__ __forceinline__ void merge_row(const MergeArgs& a, int row, int lane) {
-  constexpr int kMaxSlices = 8;
   const int n = a.n_rows;
   const float4* prow = a.part + static_cast<int64_t>(row) * a.parts_per_row;
   const int tiles_per_slice = a.vchunk / kTile;
-  float4 p[kMaxSlices];
-  if constexpr (kOne) {
+  // columns of slice c (the vocabulary's last one may be narrower; 0 past it) and its tiles
+  auto cols_of = [&](int c) { return min(a.vchunk, a.vocab - a.col0 - c * a.vchunk); };
+  auto tiles_of = [&](int c) { return c < a.n_slices ? (cols_of(c) + kTile - 1) / kTile : 0; };
+  float4 p[kSliceLoads];
+  auto load = [&](int c0) {  // the tiles of slices c0 .. c0 + 7
 #pragma unroll
-    for (int c = 0; c < kMaxSlices; ++c) {
-      const int tiles = c < a.n_slices ? (a.slice_cols[c] + kTile - 1) / kTile : 0;
-      p[c] = lane < tiles ? prow[c * tiles_per_slice + lane] : make_float4(-INFINITY, 0.f, 0.f, 0.f);
-    }
-  }
+    for (int c = 0; c < kSliceLoads; ++c)
+      p[c] = lane < tiles_of(c0 + c) ? prow[(c0 + c) * tiles_per_slice + lane]
+                                     : make_float4(-INFINITY, 0.f, 0.f, 0.f);
+  };
+  if constexpr (kOne) load(0);
   const int64_t target = a.targets[row];
   const bool labelled = target >= 0;
   const float zt_new = a.ztarget[row];  // meaningful only when the target is in this group
@@ -505,12 +530,12 @@ __device__ __forceinline__ void merge_row(const MergeArgs& a, int row, int lane)
     m = run[row]; s = run[n + row]; t = run[2 * n + row]; best = run[3 * n + row];
     zt = run[4 * n + row]; bidx = __float_as_int(run[5 * n + row]);
   }
-  auto slice = [&](int c) {
-    const int tiles = (a.slice_cols[c] + kTile - 1) / kTile;
+  auto slice = [&](int c, float4 pc) {
+    const int tiles = tiles_of(c);
     const int tile0 = c * tiles_per_slice;
     Stat acc{-INFINITY, 0.f, 0.f, 0x7fffffff};
     if constexpr (kOne) {
-      if (lane < tiles) acc = merge(acc, Stat{p[c].x, p[c].y, p[c].z, __float_as_int(p[c].w)});
+      if (lane < tiles) acc = merge(acc, Stat{pc.x, pc.y, pc.z, __float_as_int(pc.w)});
     } else {
       for (int tt = lane; tt < tiles; tt += kWave) {
         const float4 q = prow[tile0 + tt];
@@ -530,16 +555,21 @@ __device__ __forceinline__ void merge_row(const MergeArgs& a, int row, int lane)
       best = acc.m;
       bidx = acc.idx;
     }
-    const int64_t rel = target - a.slice_col0[c];
-    if (labelled && rel >= 0 && rel < a.slice_cols[c]) zt = zt_new;
+    const int64_t rel = target - (a.col0 + static_cast<int64_t>(c) * a.vchunk);
+    if (labelled && rel >= 0 && rel < cols_of(c)) zt = zt_new;
   };
   const float m_prev = m;  // the running maximum before this group
   if constexpr (kOne) {
+    for (int c0 = 0;;) {
 #pragma unroll
-    for (int c = 0; c < kMaxSlices; ++c)
-      if (c < a.n_slices) slice(c);
+      for (int c = 0; c < kSliceLoads; ++c)
+        if (c0 + c < a.n_slices) slice(c0 + c, p[c]);
+      c0 += kSliceLoads;
+      if (c0 >= a.n_slices) break;
+      load(c0);
+    }
   } else {
-    for (int c = 0; c < a.n_slices; ++c) slice(c);
+    for (int c = 0; c < a.n_slices; ++c) slice(c, float4{});
   }
   // The reference adds fp16(e^{z - m_c}) W_c into its fp32 accumulator after rescaling it by
   // e^{m_old - m_c} at every slice (solution/fused_head.py:170-182); the rescales of one group's
@@ -548,28 +578,25 @@ __device__ __forceinline__ void merge_row(const MergeArgs& a, int row, int lane)
   // fp16(e^{m_t - m_G}) in head_grad (one more fp16 rounding than the reference's P, as before),
   // so the group's columns form one plain reduction that head_grad may cut anywhere, and
   // head_combine rescales the accumulator once per group by e^{m_prev - m_G}.
-  auto factors = [&](int c) {
-      const int tiles = (a.slice_cols[c] + kTile - 1) / kTile;
-      const int tile0 = c * tiles_per_slice;
-      if constexpr (kOne) {
-        if (lane < tiles) {
-          const float mt = p[c].x;
-          a.scale[scale_index(row, tile0 + lane, a.scale_blocks)] = f2h(mt == -INFINITY ? 0.f : __expf(mt - m));
-        }
-      } else {
-        for (int tt = lane; tt < tiles; tt += kWave) {
-          const float mt = prow[tile0 + tt].x;
-          a.scale[scale_index(row, tile0 + tt, a.scale_blocks)] = f2h(mt == -INFINITY ? 0.f : __expf(mt - m));
-        }
-      }
-  };
   if (row < a.n_grad) {
     if constexpr (kOne) {
+      for (int c0 = 0; c0 < a.n_slices; c0 += kSliceLoads) {
+        if (a.n_slices > kSliceLoads) load(c0);  // a single set is still in registers
 #pragma unroll
-      for (int c = 0; c < kMaxSlices; ++c)
-        if (c < a.n_slices) factors(c);
+        for (int c = 0; c < kSliceLoads; ++c)
+          if (lane < tiles_of(c0 + c)) {
+            const float mt = p[c].x;
+            a.scale[scale_index(row, (c0 + c) * tiles_per_slice + lane, a.scale_blocks)] =
+                f2h(mt == -INFINITY ? 0.f : __expf(mt - m));
+          }
+      }
     } else {
-      for (int c = 0; c < a.n_slices; ++c) factors(c);
+      for (int c = 0; c < a.n_slices; ++c)
+        for (int tt = lane; tt < tiles_of(c); tt += kWave) {
+          const float mt = prow[c * tiles_per_slice + tt].x;
+          a.scale[scale_index(row, c * tiles_per_slice + tt, a.scale_blocks)] =
+              f2h(mt == -INFINITY ? 0.f : __expf(mt - m));
+        }
     }
   }
   if (lane == 0)
@@ -826,7 +853,7 @@ constexpr int kCus = 256;  // MI355X compute units
 // workgroups x steps per part x a 64-deep step's time with every CU busy (1.7 us, measured),
 // plus each part's partial written and read back at 5 TB/s.
 constexpr double kStepUs = 1.7, kPartialBytesPerUs = 5e6;
-constexpr int kMaxParts = 16;
+constexpr int kMaxParts = 48;  // 6 tiles (256 rows, hidden 1536) x 42 parts fill the chip
 
 struct GradPlan {
   int parts;           // parts holding work
@@ -851,6 +878,27 @@ GradPlan plan_grad(int64_t n_grad, int64_t hidden, int64_t group_cols) {
     }
   }
   return best;
+}
+
+// Slices per step of the slice loop (a step is one launch each of head_logits, head_merge,
+// head_grad and head_combine): at least `group`, and as many more as fit the bound of what a step
+// leaves behind.
+// - With gradient rows that is P (2 bytes per gradient row and column), written by head_logits and
+//   read by head_grad: 168 MiB of it stay in the 256 MiB last-level cache beside the weights. Fewer,
+//   larger launches fill the chip better (hidden 1536, vocabulary 151936, training, against five
+//   slices a step: 64 rows 514 -> 293 us, 257 681 -> 483, 517 805 -> 705, 1167 1390 -> 1285; at
+//   1843 and 2048 rows eight slices, 241 and 268 MB of P, cost 4% and 7%).
+// - Without, only the tiles' statistics (16 bytes per row and 128 columns): 64 MiB (3500 rows at a
+//   vocabulary of 151936; 64 rows 259 -> 166 us, 517 400 -> 328, 1167 733 -> 590, 2048 984 -> 963).
+int slices_per_step(int64_t n_rows, int64_t vocab, int64_t vchunk, int64_t n_grad, int group) {
+  const int64_t slices = (vocab + vchunk - 1) / vchunk;
+  const int64_t per_slice = n_grad > 0 ? n_grad * vchunk * 2 : n_rows * (vchunk / kTile) * 16;
+  const int64_t bound = int64_t{n_grad > 0 ? 168 : 64} << 20;
+  const int64_t most = std::min(
+      slices, std::max<int64_t>(group, std::min(bound / std::max<int64_t>(per_slice, 1),
+                                                ((int64_t{1} << 22) - 1) / vchunk)));
+  const int64_t steps = (slices + most - 1) / most;  // of nearly equal size: 19 slices go 10 + 9
+  return static_cast<int>(std::min(slices, std::max<int64_t>(group, (slices + steps - 1) / steps)));
 }
 
 struct Layout {
@@ -895,9 +943,11 @@ TALM_API int64_t talm_head_ce_workspace(int64_t n_rows, int64_t hidden, int64_t 
   if (n_rows < 0 || hidden < 1 || vocab < 1 || vchunk < kTile || vchunk % kTile || n_grad < 0 ||
       n_grad > n_rows || group < 1 || group > 8)
     return -1;
-  const int64_t slices = (vocab + vchunk - 1) / vchunk;
-  const int g = static_cast<int>(slices < group ? slices : group);
-  return static_cast<int64_t>(layout(n_rows, hidden, vocab, vchunk, n_grad, g).total);
+  // for either step that talm_head_ce may take
+  const int g = slices_per_step(n_rows, vocab, vchunk, n_grad, group);
+  const int few = static_cast<int>(std::min<int64_t>((vocab + vchunk - 1) / vchunk, group));
+  return static_cast<int64_t>(std::max(layout(n_rows, hidden, vocab, vchunk, n_grad, g).total,
+                                       layout(n_rows, hidden, vocab, vchunk, n_grad, few).total));
 }
 
 TALM_API int talm_head_weight_t(const uint16_t* weight, int64_t ldw, int64_t vocab,
@@ -945,8 +995,15 @@ TALM_API int talm_head_ce(const uint16_t* hidden_states, int64_t ldh, const uint
     return fail(TALM_EINVAL, "head_ce: hidden states, weight and dH must be 16-byte "
                              "aligned, the workspace 256-byte aligned");
   const int64_t slices = (vocab + vchunk - 1) / vchunk;
-  const int g = static_cast<int>(slices < group ? slices : group);
-  const Layout l = layout(n_rows, hidden, vocab, vchunk, n_grad, g);
+  // the larger step, unless its weight rows are out of a buffer load's reach or the workspace was
+  // sized for fewer rows per step (one kept for calls of several sizes)
+  int g = slices_per_step(n_rows, vocab, vchunk, n_grad, group);
+  Layout l = layout(n_rows, hidden, vocab, vchunk, n_grad, g);
+  if ((with_grad && g * vchunk * ldw * 2 >= (int64_t{1} << 31)) ||
+      workspace_bytes < static_cast<int64_t>(l.total)) {
+    g = static_cast<int>(std::min<int64_t>(slices, group));
+    l = layout(n_rows, hidden, vocab, vchunk, n_grad, g);
+  }
   if (l.ldz >= (1 << 22))
     return fail(TALM_EINVAL, "head_ce: group * vchunk = %lld columns per step, below 2^22 needed",
                 (long long)l.ldz);
@@ -980,8 +1037,9 @@ TALM_API int talm_head_ce(const uint16_t* hidden_states, int64_t ldh, const uint
     la.parts_per_row = l.parts_per_row; la.targets = targets; la.ztarget = ztarget; la.n_p = n_p;
     la.n_ttiles = (rows + LogitsShape::kBN - 1) / LogitsShape::kBN;
     la.n_tiles = la.n_ttiles * static_cast<int>((gcols + LogitsShape::kBM - 1) / LogitsShape::kBM);
-    // one workgroup per CU (a multiple of 8, one range per XCD) or one per tile, if fewer
-    int wgs = std::min(la.n_tiles, device_cus());
+    // one workgroup per CU or tile, in whole multiples of 8 (one range per XCD): rounded up, so that
+    // 246 tiles run in one round (a workgroup without a tile exits), never past the CUs
+    int wgs = std::min((la.n_tiles + kXcds - 1) / kXcds * kXcds, device_cus());
     if (wgs >= kXcds) wgs -= wgs % kXcds;
     hipLaunchKernelGGL((head_logits_kernel<LogitsShape>), dim3(static_cast<unsigned>(wgs)),
                        dim3(LogitsShape::kThreads), 0, s, la);
@@ -991,11 +1049,7 @@ TALM_API int talm_head_ce(const uint16_t* hidden_states, int64_t ldh, const uint
     ma.targets = targets; ma.ztarget = ztarget; ma.n_rows = rows;
     ma.n_grad = n_p;
     ma.n_slices = ns; ma.vchunk = static_cast<int>(vchunk);
-    for (int c = 0; c < ns; ++c) {
-      const int64_t c0 = col0 + c * vchunk;
-      ma.slice_col0[c] = static_cast<int>(c0);
-      ma.slice_cols[c] = static_cast<int>(vocab - c0 < vchunk ? vocab - c0 : vchunk);
-    }
+    ma.col0 = static_cast<int>(col0); ma.vocab = static_cast<int>(vocab);
     ma.first_slice = s0 == 0;
     ma.last_slice = s0 + ns == slices;
     ma.run = run; ma.alpha = alpha;

@@ -14,7 +14,7 @@ import pytest
 import torch
 
 from oracle import head as head_oracle
-from talm_amd import fused_head, workloads
+from talm_amd import _ops, fused_head, workloads
 from tests.test_oracle import exact_head_case
 
 pytestmark = pytest.mark.gpu
@@ -144,6 +144,47 @@ def test_head_argmax_ties_across_slices_and_groups():
     res = _run(h, w, t, vchunk=8192)
     assert res["correct"][:2 * len(pairs)].tolist() == [True, False] * len(pairs)
     assert res["best_idx"][:2 * len(pairs)].tolist() == [a for a, _ in pairs for _ in range(2)]
+
+
+@pytest.mark.parametrize("n", [1, 192, 193, 256, 257, 450])
+def test_head_steps_of_many_slices(n):
+    """Few rows take more than `group` slices per step (here all 22 of them, also more than the
+    eight whose statistics are loaded at a time) and the last token tile of 256 rows may be partly
+    empty, wavefront by wavefront (64 rows): losses, argmax and dH against the oracle, and the
+    evaluation equal to the training pass bit for bit."""
+    _case(f"head many slices n={n}")
+    h16, w16, t = exact_head_case(n, 64, 2800, 30 + n)
+    res = _run(h16, w16, t, vchunk=128)
+    _check(res, h16, w16, t, 128, what=f"n={n}")
+    dev = [torch.from_numpy(x).to(DEV) for x in (h16, w16, t)]
+    out = fused_head.head_ce(*dev, vocab_chunk=128, need_grad=False)
+    # the loss is 0 on unlabelled rows in both; rows are independent of their order
+    np.testing.assert_array_equal(out["token_loss"].cpu().numpy(), res["token_loss"])
+    np.testing.assert_array_equal(out["entropy"].cpu().numpy(), res["entropy"])
+    np.testing.assert_array_equal(out["best_idx"].cpu().numpy(), res["best_idx"])
+
+
+@pytest.mark.parametrize("n_grad", [0, 70])
+def test_head_workspace_of_the_smaller_step(n_grad):
+    """A workspace that holds `group` slices a step but not more (one kept from another call) still
+    serves: the loop takes `group` at a time, with the same losses and dH to the rescales'
+    rounding (each step's factors are rounded to fp16)."""
+    group, vchunk, vocab = 3, 128, 9 * 128
+    h16, w16, t = exact_head_case(70, 64, vocab, 50)
+    h, w, tt = [torch.from_numpy(x).to(DEV) for x in (h16, w16, t)]
+    small = _ops.head_ce_workspace_bytes(70, 64, group * vchunk, vchunk, n_grad, group)
+    assert small < _ops.head_ce_workspace_bytes(70, 64, vocab, vchunk, n_grad, group)
+    full = fused_head.head_ce(h, w, tt, vchunk, n_grad, n_grad > 0, group)
+    got = {k: torch.empty_like(v) for k, v in full.items() if v is not None}
+    ws = torch.empty(small, dtype=torch.uint8, device=DEV)
+    torch.ops.talm.head_ce(h, w, tt, vchunk, n_grad, group, got["token_loss"], got["entropy"],
+                           got["best_idx"], got["correct"], got.get("grad"), ws)
+    assert torch.equal(got["best_idx"], full["best_idx"])
+    assert torch.equal(got["token_loss"], full["token_loss"])
+    if n_grad:  # one fp16 rounding of each column's factor, one of dH
+        ref = full["grad"].double()
+        bound = 2.0 ** -10 * (ref.abs() + w.double().abs().max())
+        assert bool(((got["grad"].double() - ref).abs() <= bound).all())
 
 
 def test_head_config4_full_size_every_row():
