@@ -570,6 +570,16 @@ int talm_nf4_gemm_partials(const uint16_t* x, int64_t ldx, int64_t n_tokens, con
  * stats int64 [2] = (#i with correct[i] != 0 (bytes), #i with targets[i] >= 0). Replaces the scatter of
  * the per-token outputs and the step's metric sums (solution/patches.py:244-253).
  *
+ * talm_head_order: the rows of hidden f16 [n, hidden] (row stride ldh, a multiple of 8; hidden too)
+ * and their targets in labelled-first order: row r to dest[r] = the number of labelled rows before
+ * it (target >= 0), or n_labelled + the unlabelled rows before it; n_labelled is the exact count.
+ * out f16 [n, hidden] contiguous, targets_out, dest i64 [n]. Replaces solution/fused_head.py:290-299
+ * with the two gathers of :328-336.
+ *
+ * talm_head_restore: row r of each output is row dest[r] of its input (token_loss, entropy f32,
+ * correct, best_idx i32 [n], grad f16 [n, hidden] contiguous). Replaces the gathers back to the
+ * input order (solution/fused_head.py:374-383).
+ *
  * talm_scale_rows: out[i] = fp16(fp32(g[i]) * s), s = *grad_loss / *denom (0 when *denom is 0),
  * fp16 [n], 16-byte aligned. Replaces the head's backward (solution/fused_head.py:280-287).
  */
@@ -584,6 +594,13 @@ int talm_head_loss(const float* token_loss, const int32_t* correct, const int64_
 int talm_scatter_rows(const float* token_loss, const float* entropy, const uint8_t* correct,
                       const int64_t* targets, const int64_t* src, int64_t n, int64_t out_len,
                       float* full_loss, float* full_entropy, int64_t* stats, void* stream);
+int talm_head_order(const uint16_t* hidden, int64_t ldh, const int64_t* targets, int64_t n,
+                    int64_t hidden_size, int64_t n_labelled, uint16_t* out, int64_t* targets_out,
+                    int64_t* dest, void* stream);
+int talm_head_restore(const float* token_loss, const float* entropy, const int32_t* correct,
+                      const int32_t* best_idx, const uint16_t* grad, const int64_t* dest, int64_t n,
+                      int64_t hidden_size, float* token_loss_out, float* entropy_out,
+                      int32_t* correct_out, int32_t* best_idx_out, uint16_t* grad_out, void* stream);
 int talm_scale_rows(const uint16_t* g, int64_t n, const float* grad_loss, const float* denom,
                     uint16_t* out, void* stream);
 

@@ -66,6 +66,8 @@ SIGNATURES = {
     "talm_row_stats": [_P, _P, _I32, _I32, _P, _P],
     "talm_head_loss": [_P, _P, _P, _I64, _P, _F32, _I32, _P, _P, _P, _P],
     "talm_scatter_rows": [_P, _P, _P, _P, _P, _I64, _I64, _P, _P, _P, _P],
+    "talm_head_order": [_P, _I64, _P, _I64, _I64, _I64, _P, _P, _P, _P],
+    "talm_head_restore": [_P, _P, _P, _P, _P, _P, _I64, _I64, _P, _P, _P, _P, _P, _P],
     "talm_scale_rows": [_P, _I64, _P, _P, _P, _P],
     "talm_lora_adamw": [_P, _I32, _I64, _F32, _F32, _F32, _F32, _F32, _P, _P, _P, _P, _P, _P],
     "talm_lora_grad_norm": [_P, _I32, _I64, _P, _F32, _P, _I64, _P, _P],

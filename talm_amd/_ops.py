@@ -24,7 +24,7 @@ OPS = ("nf4_group_dequant", "nf4_group_dequant_streaming", "nf4_dequant", "rmsno
        "head_weight_t", "head_ce", "lora_down", "qkv_lora_fwd", "qkv_lora_fwd_down", "qkv_bwd_prep", "qkv_lora_bwd_dx",
        "lora_wgrad", "gemm", "gemm_ex", "attn_fwd", "attn_bwd", "attn_bwd_rope", "lora_mirror",
        "lora_adamw", "nf4_gemm", "nf4_block_scales", "nf4_group_dequant_t", "gemm_splitk",
-       "pack_rows", "row_stats", "head_loss", "scatter_rows", "scale_rows",
+       "pack_rows", "row_stats", "head_loss", "scatter_rows", "head_order", "head_restore", "scale_rows",
        "gemm_splitk_partials", "nf4_gemm_partials", "splitk_add_rmsnorm", "splitk_rmsnorm_bwd",
        "rope_table", "lora_grad_norm", "lora_adamw_clipped")
 

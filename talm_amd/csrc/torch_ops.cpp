@@ -1400,6 +1400,56 @@ void scatter_rows(const Tensor& token_loss, const Tensor& entropy, const Tensor&
         "scatter_rows");
 }
 
+// hidden fp16 [N, H] (unit column stride), targets int64 [N] -> out fp16 [N, H], targets_out and
+// dest int64 [N], labelled rows first.
+void head_order(const Tensor& hidden, const Tensor& targets, int64_t n_labelled, const Tensor& out,
+                const Tensor& targets_out, const Tensor& dest) {
+  require_fp16(hidden, "hidden");
+  require_fp16(out, "out");
+  i64_cuda(targets, "targets");
+  i64_cuda(targets_out, "targets_out");
+  i64_cuda(dest, "dest");
+  require(hidden.dim() == 2 && hidden.stride(1) == 1 && out.sizes() == hidden.sizes() &&
+              out.is_contiguous(),
+          "head_order: hidden [N, H] with unit column stride, out contiguous of its size");
+  const int64_t n = hidden.size(0);
+  require(targets.numel() == n && targets_out.numel() == n && dest.numel() == n,
+          "head_order: targets, targets_out and dest [N]");
+  check(talm_head_order(as<uint16_t>(hidden), hidden.stride(0), as<int64_t>(targets), n,
+                        hidden.size(1), n_labelled, as<uint16_t>(out), as<int64_t>(targets_out),
+                        as<int64_t>(dest), stream_of(hidden)),
+        "head_order");
+}
+
+// Row r of each output is row dest[r] of its input.
+void head_restore(const Tensor& token_loss, const Tensor& entropy, const Tensor& correct,
+                  const Tensor& best_idx, const Tensor& grad, const Tensor& dest,
+                  const Tensor& token_loss_out, const Tensor& entropy_out,
+                  const Tensor& correct_out, const Tensor& best_idx_out, const Tensor& grad_out) {
+  const int64_t n = dest.numel();
+  i64_cuda(dest, "dest");
+  for (const Tensor* t : {&token_loss, &entropy, &token_loss_out, &entropy_out}) {
+    f32_cuda(*t, "token_loss / entropy");
+    require(t->numel() == n, "head_restore: token_loss and entropy [N]");
+  }
+  for (const Tensor* t : {&correct, &best_idx, &correct_out, &best_idx_out})
+    require(t->is_cuda() && t->scalar_type() == at::kInt && t->is_contiguous() && t->numel() == n,
+            "head_restore: correct and best_idx int32 [N]");
+  require_fp16(grad, "grad");
+  require_fp16(grad_out, "grad_out");
+  require(grad.dim() == 2 && grad.size(0) == n && grad.is_contiguous() &&
+              grad_out.sizes() == grad.sizes() && grad_out.is_contiguous(),
+          "head_restore: grad [N, H] contiguous");
+  check(talm_head_restore(as<float>(token_loss), as<float>(entropy),
+                          static_cast<const int32_t*>(correct.data_ptr()),
+                          static_cast<const int32_t*>(best_idx.data_ptr()), as<uint16_t>(grad),
+                          as<int64_t>(dest), n, grad.size(1), as<float>(token_loss_out),
+                          as<float>(entropy_out), static_cast<int32_t*>(correct_out.data_ptr()),
+                          static_cast<int32_t*>(best_idx_out.data_ptr()), as<uint16_t>(grad_out),
+                          stream_of(grad)),
+        "head_restore");
+}
+
 // out = fp16(fp32(g) * (denom != 0 ? grad_loss / denom : 0)); g, out fp16 of one size.
 void scale_rows(const Tensor& g, const Tensor& grad_loss, const Tensor& denom, const Tensor& out) {
   require_fp16(g, "g");
@@ -1476,6 +1526,11 @@ TORCH_LIBRARY(talm, m) {
         "Tensor(c!) correct_bool) -> ()");
   m.def("scatter_rows(Tensor token_loss, Tensor entropy, Tensor correct, Tensor targets, "
         "Tensor src, Tensor(a!) full_loss, Tensor(b!) full_entropy, Tensor(c!) stats) -> ()");
+  m.def("head_order(Tensor hidden, Tensor targets, int n_labelled, Tensor(a!) out, "
+        "Tensor(b!) targets_out, Tensor(c!) dest) -> ()");
+  m.def("head_restore(Tensor token_loss, Tensor entropy, Tensor correct, Tensor best_idx, "
+        "Tensor grad, Tensor dest, Tensor(a!) token_loss_out, Tensor(b!) entropy_out, "
+        "Tensor(c!) correct_out, Tensor(d!) best_idx_out, Tensor(e!) grad_out) -> ()");
   m.def("scale_rows(Tensor g, Tensor grad_loss, Tensor denom, Tensor(a!) out) -> ()");
   m.def("lora_grad_norm(Tensor table, int n_tensors, int max_numel, Tensor scale, "
         "float max_norm, Tensor(a!) workspace, Tensor(b!) stats) -> ()");
@@ -1538,6 +1593,8 @@ TORCH_LIBRARY_IMPL(talm, CUDA, m) {
   m.impl("row_stats", &row_stats);
   m.impl("head_loss", &head_loss);
   m.impl("scatter_rows", &scatter_rows);
+  m.impl("head_order", &head_order);
+  m.impl("head_restore", &head_restore);
   m.impl("scale_rows", &scale_rows);
   m.impl("rope_table", &rope_table);
   m.impl("lora_grad_norm", &lora_grad_norm);

@@ -155,7 +155,7 @@ def _head_backward(ctx, grad_loss):
 
 
 def labelled_first(labelled, n_labelled):
-    """(dest, src): row r of the input goes to position dest[r] of the labelled-first order and
+    """The order that talm_head_order makes, in PyTorch. (dest, src): row r of the input goes to position dest[r] of the labelled-first order and
     reordered row i is input row src[i] (solution/fused_head.py:290-299; no host sync)."""
     n = labelled.shape[0]
     pos = torch.arange(n, device=labelled.device)
@@ -163,6 +163,14 @@ def labelled_first(labelled, n_labelled):
     dest = torch.where(labelled, seen - 1, pos - seen + n_labelled)
     src = torch.empty_like(dest).index_copy_(0, dest, pos)
     return dest, src
+
+
+def _order_rows(h16, targets, n_labelled):
+    """(hidden rows, targets) in `labelled_first`'s order and its dest, in one launch."""
+    out = torch.empty(h16.shape, dtype=torch.float16, device=h16.device)
+    rows_targets, dest = torch.empty_like(targets), torch.empty_like(targets)
+    torch.ops.talm.head_order(h16, targets, n_labelled, out, rows_targets, dest)
+    return out, rows_targets, dest
 
 
 def _fp16_weight(weight):
@@ -197,20 +205,17 @@ class FusedHeadLossVocab(torch.autograd.Function):
             if not COMPACT and 0 < n_grad < n_tokens:
                 raise ValueError("the MI355X head accumulates labelled-first rows only")
             if 0 < n_grad < n_tokens:
-                dest, src = labelled_first(targets >= 0, n_grad)
-                h16 = h16.index_select(0, src)
-                rows_targets = targets.index_select(0, src)
+                h16, rows_targets, dest = _order_rows(h16, targets, n_grad)
                 RAN["compact"] += 1
         out = head_ce(h16, w16, rows_targets, vocab_chunk, n_grad, need_grad)
         RAN["head"] += 1
         token_loss, entropy = out["token_loss"], out["entropy"]
         correct, best_idx, grad_hidden = out["correct"], out["best_idx"], out["grad"]
         if dest is not None:
-            token_loss = token_loss.index_select(0, dest)
-            entropy = entropy.index_select(0, dest)
-            correct = correct.index_select(0, dest)
-            best_idx = best_idx.index_select(0, dest)
-            grad_hidden = grad_hidden.index_select(0, dest)
+            ordered = (token_loss, entropy, correct, best_idx, grad_hidden)
+            token_loss, entropy, correct, best_idx, grad_hidden = restored = [
+                torch.empty_like(t) for t in ordered]
+            torch.ops.talm.head_restore(*ordered, dest, *restored)
         loss, denom, correct = _loss(token_loss, correct, targets, num_items)
         ctx.denom = denom
         ctx.out_dtype = hidden.dtype

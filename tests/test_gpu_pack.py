@@ -120,6 +120,37 @@ def test_scale_rows_is_the_reference_arithmetic(n, denom_value):
     assert torch.equal(out.view(torch.int16), expect.view(torch.int16))
 
 
+@pytest.mark.parametrize("n,hidden,ld", [(1, 8, 8), (8, 1536, 1536), (9, 72, 80), (65, 1544, 1544),
+                                         (2048, 1536, 1536), (16385, 64, 64), (140000, 8, 16)])
+def test_head_order_is_labelled_first(n, hidden, ld):
+    """Rows per workgroup 8 up to 16384 rows, more beyond (past 64 from 131073 rows on)."""
+    import talm_amd._ops  # noqa: F401
+    from talm_amd import fused_head
+
+    print(f"[case] head_order n={n} hidden={hidden} ld={ld}", flush=True)
+    g = torch.Generator().manual_seed(n)
+    base = torch.randn(n, ld, generator=g).half()
+    targets = torch.randint(-2, 5, (n,), generator=g)
+    labelled = targets >= 0
+    count = int(labelled.sum())
+    dest, src = fused_head.labelled_first(labelled, count)
+    h = base.cuda()[:, :hidden]
+    out, rows_targets, got = fused_head._order_rows(h, targets.cuda(), count)
+    assert torch.equal(got.cpu(), dest)
+    assert torch.equal(rows_targets.cpu(), targets[src])
+    assert torch.equal(out.cpu(), base[src, :hidden])
+    # and back
+    loss, ent = torch.rand(n, generator=g), torch.rand(n, generator=g)
+    corr = torch.randint(0, 2, (n,), generator=g, dtype=torch.int32)
+    best = torch.randint(0, 1 << 20, (n,), generator=g, dtype=torch.int32)
+    ordered = [t.cuda() for t in (loss, ent, corr, best)] + [out]
+    back = [torch.full_like(t, 77) for t in ordered]
+    torch.ops.talm.head_restore(*ordered, got, *back)
+    for t, b in zip((loss, ent, corr, best), back):
+        assert torch.equal(b.cpu(), t[dest])
+    assert torch.equal(back[4].cpu(), base[:, :hidden])
+
+
 def test_rmsnorm_backward_without_a_sum_gradient_equals_a_zero_one():
     """The add-norm backward with no gradient of the sum (the final norm) reads no ds operand:
     the same bits as the launch with a zero-filled one."""
