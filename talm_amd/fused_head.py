@@ -155,8 +155,9 @@ def _head_backward(ctx, grad_loss):
 
 
 def labelled_first(labelled, n_labelled):
-    """The order that talm_head_order makes, in PyTorch. (dest, src): row r of the input goes to position dest[r] of the labelled-first order and
-    reordered row i is input row src[i] (solution/fused_head.py:290-299; no host sync)."""
+    """The order that talm_head_order makes, in PyTorch. (dest, src): row r of the input goes to
+    position dest[r] of the labelled-first order and reordered row i is input row src[i]
+    (solution/fused_head.py:290-299; no host sync)."""
     n = labelled.shape[0]
     pos = torch.arange(n, device=labelled.device)
     seen = torch.cumsum(labelled, 0)
