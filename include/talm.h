@@ -402,7 +402,8 @@ int talm_attn_fwd(const uint16_t* q, int64_t q_stride_tok, int64_t q_stride_head
  * elements) from q, k, v, the forward's out and lse, and dout. dk / dv of
  * a KV head sum its query heads' contributions in head order (deterministic). `workspace`
  * (256-byte aligned) holds talm_attn_bwd_workspace(n_tokens, n_q_heads) bytes: rowsum(dout *
- * out), lse in base-2 units and fp32 dk / dv partials per query head. Replaces the backward of the same launches
+ * out), lse in base-2 units, fp32 dk / dv partials per query head and, in the last 256 bytes, the
+ * counter of a work queue (without these 256 bytes the call still runs, unqueued). Replaces the backward of the same launches
  * (solution/unpad.py:199-294).
  */
 int64_t talm_attn_bwd_workspace(int64_t n_tokens, int32_t n_q_heads);

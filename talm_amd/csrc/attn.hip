@@ -32,6 +32,8 @@
 // The dQ and dK / dV bodies run in one launch.
 #include "mfma_tile.h"
 
+#include <algorithm>
+
 namespace talm {
 namespace {
 
@@ -512,6 +514,9 @@ struct BwdArgs {
   int64_t n_tokens;
   float* dd;           // [Hq, n_tokens]: rowsum(dO * O)
   float* lse2;         // [Hq, n_tokens]: lse in base-2 units (lse * log2 e)
+  unsigned* counter;   // the next work item of attn_bwd_queue_kernel (null: one workgroup per item)
+  unsigned queue_wgs;  // its workgroups, each starting with the item of its own index
+  int n_seqs;
   float* dk_part;      // [Hq, n_tokens, D] fp32
   float* dv_part;      // [Hq, n_tokens, D] fp32
   uint16_t* dq;
@@ -551,6 +556,7 @@ __device__ __forceinline__ void rope_back4(float (&x)[4], float (&y)[4], const f
 __global__ __launch_bounds__(256) void attn_bwd_dot_kernel(BwdArgs a) {
   const int64_t row = (static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x) >> 4;  // t * Hq + h
   const int sub = threadIdx.x & 15;
+  if (a.counter && blockIdx.x == 0 && threadIdx.x == 0) *a.counter = a.queue_wgs;
   const int64_t rows = a.n_tokens * a.n_q_heads;
   const int64_t r = row < rows ? row : rows - 1;
   const int64_t t = r / a.n_q_heads;
@@ -627,10 +633,10 @@ __device__ __forceinline__ uint32_t slot_step(int slot) {
 
 // dQ: the forward's structure, one query row per lane (S^T = K Q^T, dP^T = V dO^T, then
 // dQ^T += K^T dS^T with K^T read transposed from the K tile); `tile` is the 32W-row query tile.
-template <int W>
-__device__ __forceinline__ void attn_bwd_dq(const BwdArgs& a, int tile, unsigned char* smem) {
+template <int W, class Done>
+__device__ __forceinline__ void attn_bwd_dq(const BwdArgs& a, int seq, int head, int tile,
+                                            unsigned char* smem, Done&& done) {
   constexpr int kRows = 32 * W;
-  const int seq = blockIdx.y, head = blockIdx.x;
   const int s0 = a.cu[seq], len = a.cu[seq + 1] - s0;
   const int q0 = tile * kRows;
   if (q0 >= len) return;
@@ -788,6 +794,7 @@ __device__ __forceinline__ void attn_bwd_dq(const BwdArgs& a, int tile, unsigned
     slot = slot == 2 ? 0 : slot + 1;
   }
 
+  done();
   __syncthreads();  // every wavefront is done with the ring: it becomes the output staging
   uint16_t* os = reinterpret_cast<uint16_t*>(smem) + wave * 32 * kKS;
   // dQ = scale * the accumulated sum; rows d = 32 j + 8 g + 4 hh + e of block j pair with the
@@ -851,11 +858,11 @@ __device__ __forceinline__ void attn_bwd_dq(const BwdArgs& a, int tile, unsigned
 // dP untransposed: keys are accumulator columns), looping over 64-row query tiles: dV^T += dO^T P
 // and dK^T += Q^T dS with Q^T and dO^T read transposed from the row-major tiles. Each slot holds
 // the Q tile, the dO tile, then each wavefront's copy of the tile's 64 lse and 64 Dd values.
-template <int W>
-__device__ __forceinline__ void attn_bwd_dkdv(const BwdArgs& a, int tile, unsigned char* smem) {
+template <int W, class Done>
+__device__ __forceinline__ void attn_bwd_dkdv(const BwdArgs& a, int seq, int head, int tile,
+                                              unsigned char* smem, Done&& done) {
   constexpr int kCols = 32 * W;  // keys per workgroup
   constexpr int kRowsT = kKeys;  // query rows per tile
-  const int seq = blockIdx.y, head = blockIdx.x;
   const int s0 = a.cu[seq], len = a.cu[seq + 1] - s0;
   const int k0 = tile * kCols;
   if (k0 >= len) return;
@@ -1056,6 +1063,7 @@ __device__ __forceinline__ void attn_bwd_dkdv(const BwdArgs& a, int tile, unsign
   // 64 rows 16 bytes each. Each wavefront stages its 32 keys x 128 columns in its own part of the
   // ring instead (rows of 132 floats: the 16 lanes of a write phase meet 16 distinct bank groups)
   // and stores whole rows, two per instruction.
+  done();
   __syncthreads();  // every wavefront is done with the ring
   constexpr int kStageLd = kD + 4;
   float* stage = reinterpret_cast<float*>(smem) + wave * 32 * kStageLd;
@@ -1103,9 +1111,72 @@ __global__ __launch_bounds__(64 * W, 1) void attn_bwd_kernel(BwdArgs a) {
   const int n_own = (len + 32 * W - 1) / (32 * W);
   if (rank >= n_own) return;  // the whole workgroup, before any barrier
   if ((blockIdx.z & 1) == 0)
-    attn_bwd_dq<W>(a, n_own - 1 - rank, smem);
+    attn_bwd_dq<W>(a, blockIdx.y, blockIdx.x, n_own - 1 - rank, smem, [] {});
   else
-    attn_bwd_dkdv<W>(a, rank, smem);
+    attn_bwd_dkdv<W>(a, blockIdx.y, blockIdx.x, rank, smem, [] {});
+}
+
+// The sum of v over the wavefront.
+__device__ __forceinline__ int wave_count(int v) {
+  return __builtin_amdgcn_readfirstlane(
+      static_cast<int>(lanes_reduce(static_cast<uint32_t>(v), [](uint32_t x, uint32_t y) { return x + y; })));
+}
+
+// The same work from a queue: one workgroup per CU takes items until none is left, the longest
+// first. With one workgroup per item the dispatcher deals them round-robin over XCDs and shader
+// engines whatever their lengths, and in order, so that a full engine holds back the others: of
+// the launch's 511 us at lengths [4096, 3001, 2222, 1531] (12 / 2 heads) a CU worked 377, of 76 us
+// at 16 rows of 128..512 tokens 51. Backward (all launches): 538 -> 463 us and 94.6 -> 82.
+//
+// An item is a (sequence, 128-token tile, dK/dV or dQ, head); its length follows the sequence's
+// tiles from there on (dK / dV: the query tiles after its keys; dQ: the key tiles before its
+// rows), so pairs (sequence, rank) go by m = tiles left, largest first. A lane holds one sequence's
+// tiles (kQueueSeqs of them); C(m) = the pairs with at least m tiles left is a sum over the lanes,
+// and an item's m is found by bisection.
+constexpr int kQueueSeqs = 64;
+template <int W>
+__global__ __launch_bounds__(64 * W, 1) void attn_bwd_queue_kernel(BwdArgs a) {
+  // the next item's index behind the ring
+  __shared__ __attribute__((aligned(1024))) unsigned char smem[kBwdLds + 16];
+  const int lane = threadIdx.x & 63;
+  const int len = lane < a.n_seqs ? a.cu[lane + 1] - a.cu[lane] : 0;
+  const int own = min((max(len, 0) + 32 * W - 1) / (32 * W), a.n_tiles);
+  const unsigned pairs = static_cast<unsigned>(wave_count(own));
+  const unsigned per_pair = 2u * static_cast<unsigned>(a.n_q_heads);
+  unsigned item = blockIdx.x;
+  for (;;) {
+    const unsigned pair = item / per_pair;
+    if (pair >= pairs) break;
+    int lo = 1, hi = a.n_tiles;  // the largest m with C(m) > pair
+    while (lo < hi) {
+      const int mid = (lo + hi + 1) >> 1;
+      if (static_cast<unsigned>(wave_count(max(own - mid + 1, 0))) > pair) lo = mid;
+      else hi = mid - 1;
+    }
+    // the pairs with exactly lo tiles left, one per sequence that has as many
+    const int nth = static_cast<int>(pair) - wave_count(max(own - lo, 0));
+    const uint64_t has = __ballot(own >= lo);
+    const bool mine = own >= lo && __popcll(has & ((uint64_t{1} << lane) - 1)) == nth;
+    const int seq = __ffsll(static_cast<unsigned long long>(__ballot(mine))) - 1;
+    const int rank = __builtin_amdgcn_readlane(own, seq) - lo;
+    const int which = static_cast<int>(item - pair * per_pair);
+    // the next item is drawn when this one's products are done, while its results go out (drawn
+    // before, the longest items would each hold back one more)
+    unsigned next = 0xffffffffu;  // past every item
+    auto draw = [&]() __attribute__((always_inline)) {
+      if (threadIdx.x == 0) next = atomicAdd(a.counter, 1u);
+    };
+    if (which < a.n_q_heads)
+      attn_bwd_dkdv<W>(a, seq, which, rank, smem, draw);
+    else
+      attn_bwd_dq<W>(a, seq, which - a.n_q_heads, lo - 1, smem, draw);
+    // the next item's counted waits start from nothing in flight, its ring from idle slots
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0) *reinterpret_cast<unsigned*>(smem + kBwdLds) = next;
+    __syncthreads();
+    item = __builtin_amdgcn_readfirstlane(*reinterpret_cast<const unsigned*>(smem + kBwdLds));
+  }
 }
 
 // dK / dV fp16 [token][kv head][d] = sum over the KV head's query heads, in head order. A
@@ -1248,12 +1319,14 @@ TALM_API int talm_attn_fwd(const uint16_t* q, int64_t q_stride_tok, int64_t q_st
   return check_launch("attn_fwd");
 }
 
+static constexpr int64_t kQueueBytes = 256;  // the work queue's counter, at the workspace's end
+
 TALM_API int64_t talm_attn_bwd_workspace(int64_t n_tokens, int32_t n_q_heads) {
   if (n_tokens < 0 || n_q_heads < 1) return -1;
   // Dd and lse2 [Hq, N] f32, then the dK and dV partials [Hq, N, D] f32 each (256-byte aligned
   // parts)
   const int64_t dd = (n_tokens * n_q_heads * 4 + 255) / 256 * 256;
-  return 2 * dd + 2 * n_tokens * n_q_heads * kD * 4;
+  return 2 * dd + 2 * n_tokens * n_q_heads * kD * 4 + kQueueBytes;
 }
 
 namespace talm {
@@ -1290,7 +1363,8 @@ int attn_bwd_impl(const uint16_t* q, int64_t q_stride_tok, int64_t q_stride_head
     return fail(TALM_EINVAL, "attn_bwd: q / k / v / dout / dq token strides must be below 2^23 elements");
   if (n_seqs > 65535 || (max_seqlen + 127) / 128 > 32767)
     return fail(TALM_EINVAL, "attn_bwd: at most 65535 sequences of at most 4194176 tokens");
-  const int64_t need = talm_attn_bwd_workspace(n_tokens, n_q_heads);
+  // (a workspace without the queue's counter is accepted: one workgroup per item then)
+  const int64_t need = talm_attn_bwd_workspace(n_tokens, n_q_heads) - kQueueBytes;
   if (workspace_bytes < need)
     return fail(TALM_EINVAL, "attn_bwd: workspace of %lld bytes, %lld needed",
                 (long long)workspace_bytes, (long long)need);
@@ -1329,13 +1403,29 @@ int attn_bwd_impl(const uint16_t* q, int64_t q_stride_tok, int64_t q_stride_head
   a.dk = dk; a.dk_tok = dk_stride_tok; a.dk_head = dk_stride_head;
   a.dv = dv; a.dv_tok = dv_stride_tok; a.dv_head = dv_stride_head;
   a.cos = rope ? cos : nullptr; a.sin = rope ? sin : nullptr; a.cs_tok = cs_stride;
+  // The queue for more than two items per CU (what there is to balance), up to one sequence per lane,
+  // where its indices fit 32 bits. Backward, grid / queue: [1500, 800] with 14 / 2 heads (532 items)
+  // 78 / 72 us, eight rows of 128..512 (672) 59 / 51, [3000] (576) 137 / 134, but [2048] (384) 82.3
+  // / 84.2, four rows of 128..512 (312) 34.9 / 35.9: finding and drawing an item costs 1-2 us.
+  const int64_t items = 2 * static_cast<int64_t>(n_q_heads) *
+                        std::min<int64_t>(n_tokens / (32 * W) + n_seqs, static_cast<int64_t>(n_seqs) * a.n_tiles);
+  a.n_seqs = n_seqs;
+  if (n_seqs <= kQueueSeqs && items > 2 * device_cus() && items < (int64_t{1} << 30) &&
+      workspace_bytes >= need + kQueueBytes) {
+    a.counter = reinterpret_cast<unsigned*>(a.dv_part + n_tokens * n_q_heads * kD);
+    a.queue_wgs = static_cast<unsigned>(std::min<int64_t>(items, device_cus()));
+  }
   const hipStream_t s = as_stream(stream);
   const int64_t rows = n_tokens * n_q_heads;
   hipLaunchKernelGGL(attn_bwd_dot_kernel, dim3(static_cast<unsigned>((rows * 16 + 255) / 256)),
                      dim3(256), 0, s, a);
-  const dim3 grid(static_cast<unsigned>(n_q_heads), static_cast<unsigned>(n_seqs),
-                  static_cast<unsigned>(2 * a.n_tiles));
-  hipLaunchKernelGGL((attn_bwd_kernel<W>), grid, dim3(64 * W), 0, s, a);
+  if (a.counter) {
+    hipLaunchKernelGGL((attn_bwd_queue_kernel<W>), dim3(a.queue_wgs), dim3(64 * W), 0, s, a);
+  } else {
+    const dim3 grid(static_cast<unsigned>(n_q_heads), static_cast<unsigned>(n_seqs),
+                    static_cast<unsigned>(2 * a.n_tiles));
+    hipLaunchKernelGGL((attn_bwd_kernel<W>), grid, dim3(64 * W), 0, s, a);
+  }
   const int64_t red = n_tokens * n_kv_heads * (rope ? kD / 8 : kD / 4);
   if (rope)
     hipLaunchKernelGGL(attn_bwd_reduce_kernel<true>, dim3(static_cast<unsigned>((red + 255) / 256)),

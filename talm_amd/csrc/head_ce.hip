@@ -488,19 +488,6 @@ struct MergeArgs {
 
 constexpr int kSliceLoads = 8;  // slices whose tiles a lane of head_merge holds at a time
 
-// v combined over the wavefront's 64 lanes, in every lane: two quad permutes and two mirrors inside
-// each row of 16 (VALU operands, no LDS permute), then the rows.
-template <class Op>
-__device__ __forceinline__ uint32_t lanes_reduce(uint32_t v, Op op) {
-  v = op(v, static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(v), 0xb1, 0xf, 0xf, true)));
-  v = op(v, static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(v), 0x4e, 0xf, 0xf, true)));
-  v = op(v, static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(v), 0x141, 0xf, 0xf, true)));
-  v = op(v, static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(v), 0x140, 0xf, 0xf, true)));
-  const auto r16 = __builtin_amdgcn_permlane16_swap(v, v, false, false);
-  v = op(r16[0], r16[1]);
-  const auto r32 = __builtin_amdgcn_permlane32_swap(v, v, false, false);
-  return op(r32[0], r32[1]);
-}
 __device__ __forceinline__ float lanes_max(float v) {
   return __uint_as_float(lanes_reduce(__float_as_uint(v), [](uint32_t a, uint32_t b) {
     return __float_as_uint(fmaxf(__uint_as_float(a), __uint_as_float(b)));

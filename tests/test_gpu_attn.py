@@ -156,6 +156,39 @@ def test_attention_backward_with_the_rotary_backward_folded_in(lengths, seed):
     _close("dv", dv, r_dv, 4e-3)
 
 
+@pytest.mark.parametrize("lengths,hq,hkv", [
+    ([0, 1, 128, 129, 700, 1500, 0, 333], 12, 2),      # empty sequences, tile edges
+    ([7 * i % 300 for i in range(64)], 12, 2),         # one sequence per lane
+    ([7 * i % 300 for i in range(65)], 12, 2),         # one more: no queue
+    ([2305], 16, 8),                                   # 608 items: just above two per CU of 256
+])
+def test_attention_backward_from_the_queue(lengths, hq, hkv):
+    """The same workgroups' work whether drawn from the queue or launched one by one (a workspace
+    without the queue's counter): the same bits, every element written, twice in a row."""
+    import talm_amd._ops  # noqa: F401
+    from talm_amd import _ops
+
+    print(f"[case] attention queue seqs={len(lengths)} heads={hq}/{hkv}", flush=True)
+    n = sum(lengths)
+    g = torch.Generator().manual_seed(n)
+    q, dout = (torch.randn(n, hq, D, generator=g).half().cuda() for _ in range(2))
+    k, v = (torch.randn(n, hkv, D, generator=g).half().cuda() for _ in range(2))
+    cu = torch.tensor([0] + lengths).cumsum(0).to("cuda", torch.int32)
+    out = torch.empty_like(q)
+    lse = torch.empty(hq, n, dtype=torch.float32, device="cuda")
+    torch.ops.talm.attn_fwd(q, k, v, cu, max(lengths), D ** -0.5, out, lse)
+    size = _ops.attn_bwd_workspace_bytes(n, hq)
+    runs = []
+    for nbytes in (size - 256, size, size):
+        ws = torch.full((nbytes,), 0xff, dtype=torch.uint8, device="cuda")
+        grads = [torch.full_like(t, float("nan")) for t in (q, k, v)]
+        torch.ops.talm.attn_bwd(q, k, v, out, dout, lse, cu, max(lengths), D ** -0.5, *grads, ws)
+        runs.append(grads)
+    for grads in runs:
+        for got, ref in zip(grads, runs[0]):
+            assert not got.isnan().any() and torch.equal(got, ref)
+
+
 def test_attention_rope_backward_rejects_bad_tables():
     import talm_amd._ops  # noqa: F401
     from talm_amd import _ops
