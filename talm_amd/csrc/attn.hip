@@ -69,7 +69,9 @@ struct FwdArgs {
   const int32_t* cu;
   int group;          // query heads per KV head
   int head_chunks;    // workgroups per KV head (group / heads per workgroup)
-  int rank_x;         // the grid's axes: (chunk, sequence, rank), or (rank, chunk, sequence)
+  int list_tiles;     // > 0: the grid is list_pair's list x chunks, its sequences of at most this many tiles
+  int n_seqs, chunks;
+  int rank_x;         // else the grid's axes: (chunk, sequence, rank), or (rank, chunk, sequence)
   float scale_log2;   // softmax scale * log2(e)
   uint16_t* out;
   int64_t o_tok, o_head;
@@ -242,6 +244,31 @@ __device__ __forceinline__ void ring2(int n, Issue&& issue, Body&& body) {
   }
 }
 
+// The sum of v over the wavefront.
+__device__ __forceinline__ int wave_count(int v) {
+  return __builtin_amdgcn_readfirstlane(
+      static_cast<int>(lanes_reduce(static_cast<uint32_t>(v), [](uint32_t x, uint32_t y) { return x + y; })));
+}
+
+// The work of up to 64 sequences, longest first: a lane holds the tiles `own` of one sequence, and the
+// pairs (sequence, m), 1 <= m <= own, go by m, largest first, and within one m by sequence. Returns
+// the m of pair `pair` (below the sum of own) and its sequence. C(m), the pairs with at least m, is a
+// sum over the lanes, so m <= m_max is found by bisection.
+constexpr int kListSeqs = 64;
+__device__ __forceinline__ int list_pair(int own, int m_max, unsigned pair, int lane, int& seq) {
+  int lo = 1, hi = m_max;  // the largest m with C(m) > pair
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (static_cast<unsigned>(wave_count(max(own - mid + 1, 0))) > pair) lo = mid;
+    else hi = mid - 1;
+  }
+  const int nth = static_cast<int>(pair) - wave_count(max(own - lo, 0));
+  const uint64_t has = __ballot(own >= lo);
+  const bool mine = own >= lo && __popcll(has & ((uint64_t{1} << lane) - 1)) == nth;
+  seq = __ffsll(static_cast<unsigned long long>(__ballot(mine))) - 1;
+  return lo;
+}
+
 // Forward, one workgroup per (sequence, H query heads of one KV head, 32 * (4 / H) query rows):
 // S groups of four wavefronts, each wavefront a head and 32 query rows, group g the key tiles g,
 // g + S, ... of 64 keys through a two-slot ring of its own.
@@ -256,7 +283,7 @@ __device__ __forceinline__ void ring2(int n, Issue&& issue, Body&& body) {
 // VALU busy together (a probe's MFMA + exponential loop), and the K / V reads from LDS.
 // Against one workgroup of six or eight wavefronts per CU on 32 query rows (128 KiB of LDS, K
 // operands waited for one by one): 16 rows of 128..512 tokens 36.2 -> 19.9 us, 16 of 1..1024 72.4 ->
-// 39.3, [4096, 3001, 2222, 1531] 187 -> 132 us (543 -> 769 TF/s), config 2's four rows 13.7 -> 13.0.
+// 39.3, [4096, 3001, 2222, 1531] 187 -> 132 us (543 -> 769 TF/s, 840 in the order of list_pair), config 2's four rows 13.7 -> 13.0.
 // Not kept: the next tile's S^T issued between this one's exponentials and P V (127 against 119 us
 // for 8 rows of 2048: 253 registers, the same clock), s_setprio around the MFMAs (no change).
 // S = 2 where it does not: the longest workgroup's chain of key tiles sets the time (about 1.1 us
@@ -272,13 +299,24 @@ __global__ __launch_bounds__(256 * S, 2) void attn_fwd_kernel(FwdArgs a) {
   static_assert(S <= 2 && kMerge + kStage <= S * kRing, "merge and output staging reuse the rings");
   __shared__ __attribute__((aligned(1024))) unsigned char smem[S * kRing];
 
-  const int rank = static_cast<int>(a.rank_x ? blockIdx.x : blockIdx.z);
-  const int chunk = static_cast<int>(a.rank_x ? blockIdx.y : blockIdx.x);
-  const int seq = static_cast<int>(a.rank_x ? blockIdx.z : blockIdx.y);
+  int chunk, seq, tile;
+  if (a.list_tiles) {
+    const int l = threadIdx.x & 63;
+    const int ll = l < a.n_seqs ? a.cu[l + 1] - a.cu[l] : 0;
+    const int own = min((max(ll, 0) + kRows - 1) / kRows, a.list_tiles);
+    const unsigned pair = blockIdx.x / a.chunks;
+    chunk = static_cast<int>(blockIdx.x - pair * a.chunks);
+    if (pair >= static_cast<unsigned>(wave_count(own))) return;
+    tile = list_pair(own, a.list_tiles, pair, l, seq) - 1;
+  } else {
+    const int rank = static_cast<int>(a.rank_x ? blockIdx.x : blockIdx.z);
+    chunk = static_cast<int>(a.rank_x ? blockIdx.y : blockIdx.x);
+    seq = static_cast<int>(a.rank_x ? blockIdx.z : blockIdx.y);
+    tile = (a.cu[seq + 1] - a.cu[seq] + kRows - 1) / kRows - 1 - rank;  // every sequence's longest tiles first
+    if (tile < 0) return;  // the whole workgroup, before any barrier
+  }
   const int kvh = chunk / a.head_chunks, hc = chunk % a.head_chunks;
   const int s0 = a.cu[seq], len = a.cu[seq + 1] - s0;
-  const int tile = (len + kRows - 1) / kRows - 1 - rank;  // every sequence's longest tiles first
-  if (tile < 0) return;  // the whole workgroup, before any barrier
   const int q0 = tile * kRows;
   const int tid = threadIdx.x, lane = tid & 63;
   // the wavefront index in a scalar register: everything the branches, loop bounds and the
@@ -1116,12 +1154,6 @@ __global__ __launch_bounds__(64 * W, 1) void attn_bwd_kernel(BwdArgs a) {
     attn_bwd_dkdv<W>(a, blockIdx.y, blockIdx.x, rank, smem, [] {});
 }
 
-// The sum of v over the wavefront.
-__device__ __forceinline__ int wave_count(int v) {
-  return __builtin_amdgcn_readfirstlane(
-      static_cast<int>(lanes_reduce(static_cast<uint32_t>(v), [](uint32_t x, uint32_t y) { return x + y; })));
-}
-
 // The same work from a queue: one workgroup per CU takes items until none is left, the longest
 // first. With one workgroup per item the dispatcher deals them round-robin over XCDs and shader
 // engines whatever their lengths, and in order, so that a full engine holds back the others: of
@@ -1130,10 +1162,7 @@ __device__ __forceinline__ int wave_count(int v) {
 //
 // An item is a (sequence, 128-token tile, dK/dV or dQ, head); its length follows the sequence's
 // tiles from there on (dK / dV: the query tiles after its keys; dQ: the key tiles before its
-// rows), so pairs (sequence, rank) go by m = tiles left, largest first. A lane holds one sequence's
-// tiles (kQueueSeqs of them); C(m) = the pairs with at least m tiles left is a sum over the lanes,
-// and an item's m is found by bisection.
-constexpr int kQueueSeqs = 64;
+// rows), the m of list_pair.
 template <int W>
 __global__ __launch_bounds__(64 * W, 1) void attn_bwd_queue_kernel(BwdArgs a) {
   // the next item's index behind the ring
@@ -1147,17 +1176,8 @@ __global__ __launch_bounds__(64 * W, 1) void attn_bwd_queue_kernel(BwdArgs a) {
   for (;;) {
     const unsigned pair = item / per_pair;
     if (pair >= pairs) break;
-    int lo = 1, hi = a.n_tiles;  // the largest m with C(m) > pair
-    while (lo < hi) {
-      const int mid = (lo + hi + 1) >> 1;
-      if (static_cast<unsigned>(wave_count(max(own - mid + 1, 0))) > pair) lo = mid;
-      else hi = mid - 1;
-    }
-    // the pairs with exactly lo tiles left, one per sequence that has as many
-    const int nth = static_cast<int>(pair) - wave_count(max(own - lo, 0));
-    const uint64_t has = __ballot(own >= lo);
-    const bool mine = own >= lo && __popcll(has & ((uint64_t{1} << lane) - 1)) == nth;
-    const int seq = __ffsll(static_cast<unsigned long long>(__ballot(mine))) - 1;
+    int seq;
+    const int lo = list_pair(own, a.n_tiles, pair, lane, seq);
     const int rank = __builtin_amdgcn_readlane(own, seq) - lo;
     const int which = static_cast<int>(item - pair * per_pair);
     // the next item is drawn when this one's products are done, while its results go out (drawn
@@ -1296,7 +1316,7 @@ TALM_API int talm_attn_fwd(const uint16_t* q, int64_t q_stride_tok, int64_t q_st
   const unsigned chunks = static_cast<unsigned>(n_q_heads / h), seqs = static_cast<unsigned>(n_seqs);
   const unsigned ranks = static_cast<unsigned>((static_cast<int64_t>(max_seqlen) + rows - 1) / rows);
   a.rank_x = ranks > 65535;
-  const dim3 grid = a.rank_x ? dim3(ranks, chunks, seqs) : dim3(chunks, seqs, ranks);
+  dim3 grid = a.rank_x ? dim3(ranks, chunks, seqs) : dim3(chunks, seqs, ranks);
   // Split the key tiles (S = 2) where the longest workgroup's chain, not the chip, sets the time:
   // the workgroups (estimated: the lengths are on the device) fit one round, one per CU, and the
   // chain is at least 8 tiles; or they fit two rounds and the chain is long enough (16 tiles) to
@@ -1306,6 +1326,19 @@ TALM_API int talm_attn_fwd(const uint16_t* q, int64_t q_stride_tok, int64_t q_st
   const int64_t wgs = (n_tokens + static_cast<int64_t>(n_seqs) * rows / 2) / rows * chunks;
   const int64_t cus = device_cus(), chain = (static_cast<int64_t>(max_seqlen) + kKeys - 1) / kKeys;
   const bool split = wgs <= cus ? chain >= 8 : wgs <= 2 * cus && chain >= 16;
+  // Workgroups by list_pair's list, longest first over all sequences, where they exceed a round (two
+  // per CU) and the sequences differ in length (an eighth of the rectangle empty): round-robin over
+  // XCDs by sequence, the longest sequences' workgroups meet on some of them. Grid / list: 16 rows of
+  // 1..1024 40.8 / 34.9 us, [4096, 3001, 2222, 1531] 135 / 120; but eight of 1024 38.7 / 40.8 and of
+  // 2048 119 / 121.5, 16 rows of 128..512 (one round) 19.0 / 20.0: finding a tile costs about 0.5 us.
+  const int64_t items = std::min<int64_t>(n_tokens / rows + n_seqs, static_cast<int64_t>(n_seqs) * ranks) * chunks;
+  if (n_seqs <= kListSeqs && wgs > 2 * cus && 8 * n_tokens < 7 * static_cast<int64_t>(n_seqs) * max_seqlen &&
+      items < (int64_t{1} << 30)) {
+    a.n_seqs = n_seqs;
+    a.chunks = chunks;
+    a.list_tiles = static_cast<int>(ranks);
+    grid = dim3(static_cast<unsigned>(items));
+  }
   const hipStream_t s = as_stream(stream);
 #define TALM_ATTN_FWD(H)                                                                         \
   if (split)                                                                                     \
@@ -1410,7 +1443,7 @@ int attn_bwd_impl(const uint16_t* q, int64_t q_stride_tok, int64_t q_stride_head
   const int64_t items = 2 * static_cast<int64_t>(n_q_heads) *
                         std::min<int64_t>(n_tokens / (32 * W) + n_seqs, static_cast<int64_t>(n_seqs) * a.n_tiles);
   a.n_seqs = n_seqs;
-  if (n_seqs <= kQueueSeqs && items > 2 * device_cus() && items < (int64_t{1} << 30) &&
+  if (n_seqs <= kListSeqs && items > 2 * device_cus() && items < (int64_t{1} << 30) &&
       workspace_bytes >= need + kQueueBytes) {
     a.counter = reinterpret_cast<unsigned*>(a.dv_part + n_tokens * n_q_heads * kD);
     a.queue_wgs = static_cast<unsigned>(std::min<int64_t>(items, device_cus()));

@@ -88,6 +88,17 @@ def test_attention_matches_per_row_causal_sdpa(lengths, strided, seed):
 
 
 @pytest.mark.parametrize("lengths,hq,hkv,seed", [
+    ([1, 2000, 64, 65, 700, 1500, 1, 1111], 12, 2, 21),   # one grid axis, 64-row tiles, mixed lengths
+    ([1024, 33, 128, 129, 900, 1, 800, 1900], 16, 16, 22),      # 128-row tiles
+    ([300] + [9 * i % 250 + 1 for i in range(63)], 16, 4, 23),  # 64 sequences, 32-row tiles
+])
+def test_attention_listed_longest_first(lengths, hq, hkv, seed):
+    """More workgroups than a round over sequences of different length: taken from the list."""
+    print(f"[case] attention listed seqs={len(lengths)} heads={hq}/{hkv} seed={seed}", flush=True)
+    _run(lengths, False, seed, hq, hkv)
+
+
+@pytest.mark.parametrize("lengths,hq,hkv,seed", [
     ([2048, 31], 12, 2, 11),       # few workgroups, a long chain: the key tiles split in two
     ([449, 64, 1], 4, 1, 12),      # four heads per workgroup, split (8 key tiles), one-tile rows
     ([448, 33], 4, 1, 13),         # the same below the split's chain length
