@@ -112,6 +112,31 @@ def test_attention_over_head_groups_and_key_splits(lengths, hq, hkv, seed):
     _run(lengths, True, seed, hq, hkv)
 
 
+@pytest.mark.parametrize("n,pos", [(256, 64), (256, 200), (600, 70), (600, 255)])
+def test_attention_largest_weight_of_the_first_tiles_is_exact(n, pos):
+    """Every score is 0 except key `pos`'s 5 (7.2 in log2 units, below the lazy rescale), and v is 0
+    except at that key: out = v e^5 / (e^5 + i). With the key's weight held as 1 its product is
+    exact, and what remains is the fp16 rounding of the output (2^-11) and that of an fp32 sum of n
+    terms; as e^5 relative to an earlier reference it adds fp16's error of 148.41, 2.6e-4."""
+    import talm_amd._ops  # noqa: F401
+
+    g = torch.Generator("cpu").manual_seed(n + pos)
+    q, k, v = torch.zeros(n, 1, D), torch.zeros(n, 1, D), torch.zeros(n, 1, D)
+    q[:, 0, 0] = 1.0
+    k[pos, 0, 0] = 5.0
+    v[pos, 0] = (1 + torch.rand(D, generator=g)).half().float()
+    cu = torch.tensor([0, n], dtype=torch.int32).cuda()
+    out = torch.empty(n, 1, D, dtype=torch.float16, device="cuda")
+    lse = torch.empty(1, n, dtype=torch.float32, device="cuda")
+    torch.ops.talm.attn_fwd(q.half().cuda(), k.half().cuda(), v.half().cuda(), cu, n, 1.0, out, lse)
+    rows = torch.arange(pos, n, dtype=torch.float64)
+    ref = v[pos, 0].double() * (math.exp(5) / (math.exp(5) + rows))[:, None]
+    err = ((out[pos:, 0].double().cpu() - ref) / ref).abs().max().item()
+    print(f"[attn] relative error {err:.3e}", flush=True)
+    assert err <= 2.0 ** -11 + n * 2.0 ** -24
+    assert not out[:pos].any()
+
+
 def _rotate_back(dy, cos, sin):
     """The gradient of x -> x cos + rotate_half(x) sin (transformers' apply_rotary_pos_emb on one
     [N, H, 128] tensor, fp32 CPU) at dy, by autograd: the rotary backward the fused kernel folds
