@@ -137,8 +137,6 @@ __device__ __forceinline__ half8_t read16_untracked(uint32_t addr, int off) {
   asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(r) : "v"(addr), "n"(off));
   return r;
 }
-// Wait until at most n LDS operations are in flight (they return in order); the registers count
-// as rewritten here.
 __device__ __forceinline__ f32x4_t read_f4_untracked(uint32_t addr, int off) {
   f32x4_t r;
   asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(r) : "v"(addr), "n"(off));
@@ -148,8 +146,14 @@ __device__ __forceinline__ f32x4_t read_f4_untracked(uint32_t addr, int off) {
 __device__ __forceinline__ void lgkm_landed(f32x4_t (&r)[4]) {
   asm volatile("" : "+v"(r[0]), "+v"(r[1]), "+v"(r[2]), "+v"(r[3]));
 }
+// Wait until at most n LDS operations are in flight (they return in order); the registers count
+// as rewritten here. n is at most 14: the counter's field has four bits, and its largest value, 15,
+// means no wait.
 __device__ __forceinline__ void lgkm_wait(int n, half8_t& r) {
   asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(r) : "n"(n));
+}
+__device__ __forceinline__ void lgkm_wait(int n, half8_t& r, half8_t& q) {
+  asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(r), "+v"(q) : "n"(n));
 }
 __device__ __forceinline__ void lgkm_wait(int n, half4_t& r, half4_t& q) {
   asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(r), "+v"(q) : "n"(n));
@@ -1013,11 +1017,13 @@ __device__ __forceinline__ void attn_bwd_dkdv(const BwdArgs& a, int seq, int hea
 #pragma unroll
     for (int s = 0; s < 8; ++s) {
       const int x = 2 * (s & 3);
-      // outstanding behind the operand: s < 4: the other row reads and the 8 lse / Dd reads, 15;
-      // then the other row reads and, from s = 5 on, 4 transposed reads per step
-      lgkm_wait(s < 4 ? 15 : (7 - 2 * (s - 4)) + (kPrev ? 4 * (s - 4) : 0), f[x]);
+      // outstanding behind the operands: s < 4: the other row reads and the 8 lse / Dd reads, 14
+      // behind the pair (15, the field's largest value, would be no wait); then the other row
+      // reads and, from s = 5 on, 4 transposed reads per step
+      if (s < 4) lgkm_wait(14, f[x], f[x + 1]);
+      else lgkm_wait((7 - 2 * (s - 4)) + (kPrev ? 4 * (s - 4) : 0), f[x]);
       sc = __builtin_amdgcn_mfma_f32_32x32x16_f16(f[x], kf[s], sc, 0, 0, 0);
-      lgkm_wait(s < 4 ? 14 : (6 - 2 * (s - 4)) + (kPrev ? 4 * (s - 4) : 0), f[x + 1]);
+      if (s >= 4) lgkm_wait((6 - 2 * (s - 4)) + (kPrev ? 4 * (s - 4) : 0), f[x + 1]);
       dp = __builtin_amdgcn_mfma_f32_32x32x16_f16(f[x + 1], vf[s], dp, 0, 0, 0);
       __builtin_amdgcn_sched_barrier(0);
       if (s < 4) {

@@ -11,7 +11,8 @@ by the register allocator.
 `violations(body)` scans a kernel body in program order. It keeps the outstanding LGKM operations
 (LDS and scalar-memory loads) and retires them at each `s_waitcnt lgkmcnt(N)`: LDS operations
 return in order, so an LDS read is complete once more than N LDS operations were issued from it
-on; scalar loads may return out of order and are retired only by `lgkmcnt(0)`. Any other
+on; scalar loads may return out of order and are retired only by `lgkmcnt(0)`. The field has four
+bits: `lgkmcnt(15)` is "do not wait" and retires nothing, however many reads are in flight. Any other
 instruction that names a VGPR / AGPR of a read still outstanding is reported. The scan is linear
 (labels do not reset the state), so it is conservative at control-flow joins.
 """
@@ -54,7 +55,7 @@ def violations(body):
                 n = int(m.group(1))
                 if n == 0:
                     pending = []
-                else:
+                elif n < 15:
                     keep = []
                     for j, entry in enumerate(pending):
                         later_ds = sum(1 for e in pending[j:] if e[0] == "ds")

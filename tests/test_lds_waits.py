@@ -1,6 +1,6 @@
 """The attention kernels read LDS through inline assembly the compiler does not track
-(talm_amd/csrc/attn.hip: read_tr_untracked, read_f4_untracked) and wait for the results
-themselves (lgkm_wait8, lgkm_wait_f4). Nothing may touch those destination registers before the
+(talm_amd/csrc/attn.hip: read_tr_untracked, read16_untracked, read_f4_untracked) and wait for the
+results themselves (lgkm_wait, lgkm_wait8). Nothing may touch those destination registers before the
 wait, not even a copy the register allocator might insert between the asm blocks. This checks
 the gfx950 assembly of every kernel with such reads (and of the other LDS-heavy kernels, whose
 reads the compiler tracks) with tests/lds_waits.py, after first checking that the scan catches
@@ -31,6 +31,10 @@ def test_scan_catches_an_early_use():
     two = ("ds_read_b128 v[8:11], v1\nds_read_b128 v[12:15], v2\ns_waitcnt lgkmcnt(1)\n"
            "v_mov_b32 v20, v8\nv_mov_b32 v21, v12\n")
     assert [ins for _, ins, _ in violations(two)] == ["v_mov_b32 v21, v12"]
+    # lgkmcnt(15) is the field's "no wait", even with more than 15 reads in flight
+    many = "".join(f"ds_read_b32 v{r}, v0\n" for r in range(10, 26))
+    assert len(violations(many + "s_waitcnt lgkmcnt(15)\nv_mov_b32 v1, v10\n")) == 1
+    assert violations(many + "s_waitcnt lgkmcnt(14)\nv_add_f32 v1, v10, v11\n") == []
     # a scalar load may return before an earlier LDS read: lgkmcnt(1) after both completes
     # neither for sure
     smem = ("ds_read_b64 v[2:3], v0\ns_load_dword s4, s[0:1], 0x0\ns_waitcnt lgkmcnt(1)\n"
@@ -75,7 +79,7 @@ def _device_asm(source):
 
 
 @pytest.mark.parametrize("source,pattern", [
-    ("attn.hip", r"attn_(fwd|bwd)_kernel"),
+    ("attn.hip", r"attn_(fwd|bwd|bwd_queue)_kernel"),
     ("head_ce.hip", r"head_(logits|grad)_kernel"),
     ("qkv.hip", r"proj_ext_kernel"),
     ("w4gemm.hip", r"w4_gemm_kernel"),
@@ -95,7 +99,7 @@ def test_no_ring_waits_for_its_prefetch(source, pattern):
 
 
 @pytest.mark.parametrize("source,pattern,untracked", [
-    ("attn.hip", r"attn_(fwd|bwd)_kernel", True),
+    ("attn.hip", r"attn_(fwd|bwd|bwd_queue)_kernel", True),
     ("w4gemm.hip", r"w4_gemm_kernel", False),
     ("head_ce.hip", r"head_(logits|grad)_kernel", False),
 ])
