@@ -15,16 +15,16 @@
 //                 that reaches global memory).
 //   head_merge    one wavefront per row folds the tiles of each slice, in column order, into the
 //                 running statistics exactly as the reference's per-slice update; for labelled
-//                 rows it writes the per-tile factors fp16(e^{m_t - m_G}) against the running max
-//                 m_G after the group and the accumulator's rescale e^{m_prev - m_G}; after the
+//                 rows it writes the per-tile factors fp16(2^14 e^{m_t - m_G}) against the running
+//                 max m_G after the group and the accumulator's rescale e^{m_prev - m_G}; after the
 //                 last slice it writes token loss, entropy, argmax and correctness.
-//   head_grad     Y = P W over the group's columns, cut into K parts that fill the chip, against
-//                 the transposed weight W^T [hidden, vocab] so that both operands are
-//                 k-contiguous; P = fp16(P_t e^{m_t - m_G}) is formed on the A fragments between
-//                 LDS and the MFMAs. The reference's per-slice rescales e^{m_old - m_c} of its
-//                 accumulator telescope over a group into e^{m_c - m_G}, so this is its
-//                 accumulator update up to one more fp16 rounding of P.
-//   head_combine  acc = e^{m_prev - m_G} acc + the parts' sum, and after the last group
+//   head_grad     Y = 2^14 P W over the group's columns, cut into K parts that fill the chip, the
+//                 weight's rows read as they lie; 2^14 P = fp16(P_t 2^14 e^{m_t - m_G}) is formed on
+//                 the A fragments between LDS and the MFMAs. The reference's per-slice rescales
+//                 e^{m_old - m_c} of its accumulator telescope over a group into e^{m_c - m_G}, so
+//                 this is its accumulator update up to two more fp16 roundings (the factor's and
+//                 the product's) of each P, relative to it down to e^{m_t - m_G} = 2^-28.
+//   head_combine  acc = e^{m_prev - m_G} acc + 2^-14 the parts' sum, and after the last group
 //                 dH = acc / s - W16[target] in fp16.
 // The full [N, V] logits never exist, only P for the gradient rows and one group's columns.
 //
@@ -455,7 +455,17 @@ __global__ __launch_bounds__(S::kThreads, 1) void head_logits_kernel(LogitsArgs 
 // ------------------------------------------------------------------------------------------
 // Running statistics, one wavefront per row, over the slices of one group.
 // ------------------------------------------------------------------------------------------
-// Factor of labelled row r and the group's 128-column tile t, e^{m_t - m_c} in fp16, where it
+// A tile's factors are stored times 2^14 (and the parts' sum is taken times 2^-14, exactly): a row
+// with a confident prediction has all its other tiles at e^{m_t - m_G} of 2^-20 and less, which in
+// fp16 would be subnormal, with a few bits or none. P_t <= 1, so the scaled product is at most 2^14.
+// Largest error of dH of six such rows (2-norm, against 64 bits; vocabulary 151936, the target 18 up on
+// logits of std 1.5, weight rows with a common mean) without / with the scale: target in the last
+// slice 7.7e-2 / 2.8e-4 with the vocabulary in one step, 1.4e-2 / 2.8e-4 in steps of five slices; in
+// the first slice 0.50 / 9.7e-3 and 0.50 / 2.5e-3 (a row of p = 0.9997; what is left are the fp32 sums
+// around W[target]). 2048 rows 1997 / 2000 us.
+constexpr float kFactorScale = 16384.f;
+
+// Factor of labelled row r and the group's 128-column tile t, 2^14 e^{m_t - m_G} in fp16, where it
 // sits for head_grad: 128-row blocks b = r / 128 of [tile][block][128] halfs, and inside a block
 // the four rows r % 32 + 32 i (i < 4) next to each other, so that one 8-byte load gives a lane of
 // a 128-row wavefront the factors of its four A-fragment rows.
@@ -600,15 +610,15 @@ __device__ __forceinline__ void merge_row(const MergeArgs& a, int row, int lane,
   // e^{m_old - m_c} at every slice (solution/fused_head.py:170-182); the rescales of one group's
   // slices telescope, so the group's contribution is sum_c e^{m_c - m_G} fp16(e^{z - m_c}) W_c with
   // m_G the running maximum after the group. Here each tile's P_t = fp16(e^{z - m_t}) is scaled by
-  // fp16(e^{m_t - m_G}) in head_grad (one more fp16 rounding than the reference's P, as before),
-  // so the group's columns form one plain reduction that head_grad may cut anywhere, and
-  // head_combine rescales the accumulator once per group by e^{m_prev - m_G}.
+  // fp16(2^14 e^{m_t - m_G}) in head_grad (kFactorScale; two more fp16 roundings than the
+  // reference's P), so the group's columns form one plain reduction that head_grad may cut
+  // anywhere, and head_combine rescales the accumulator once per group by e^{m_prev - m_G}.
   //
   // The workgroup's four rows lie 32 apart: their factors of one tile are adjacent (scale_index) and
   // go out together, 8 bytes per tile, from LDS (four 2-byte stores, each to a line of its own,
   // before).
   auto factor = [&](float mt) {
-    return real && row < a.n_grad ? f2h(mt == -INFINITY ? 0.f : __expf(mt - m)) : uint16_t{0};
+    return real && row < a.n_grad ? f2h(mt == -INFINITY ? 0.f : kFactorScale * __expf(mt - m)) : uint16_t{0};
   };
   const int base = row & ~96;  // the workgroup's first row
   if (base < a.n_grad) {       // the same in its four wavefronts
@@ -667,8 +677,8 @@ __global__ __launch_bounds__(kThreads) void head_merge_kernel(MergeArgs a) {
 // ------------------------------------------------------------------------------------------
 // GEMM2: Y_p[r][h] = sum_j P[r][j] W^T[h][col0 + j] over part p of the group's columns (a range of
 // whole 64-column steps; the group's slices lie side by side in P and in W^T), for the first
-// n_grad rows (the labelled rows, put first by the caller); P = fp16(P_t e^{m_t - m_G}) from
-// head_logits' P_t and head_merge's factors. The group's K steps are cut into `parts` equal
+// n_grad rows (the labelled rows, put first by the caller); P = fp16(P_t 2^14 e^{m_t - m_G}) from
+// head_logits' P_t and head_merge's factors (so Y is 2^14 times the group's contribution). The group's K steps are cut into `parts` equal
 // ranges so that (row tiles x hidden tiles x parts) workgroups fill the chip whatever the
 // number of labelled rows.
 // ------------------------------------------------------------------------------------------
@@ -770,7 +780,7 @@ __global__ __launch_bounds__(S::kThreads, S::kPerCu) void head_grad_kernel(GradA
 }
 
 // ------------------------------------------------------------------------------------------
-// acc = e^{m_prev - m_G} acc + sum_p Y_p (parts in order); after the last group dH = acc / s -
+// acc = e^{m_prev - m_G} acc + 2^-14 sum_p Y_p (parts in order); after the last group dH = acc / s -
 // W[target]. One thread per 4 hidden columns of one row.
 // ------------------------------------------------------------------------------------------
 struct CombineArgs {
@@ -826,6 +836,8 @@ __global__ __launch_bounds__(kThreads) void head_combine_kernel(CombineArgs a) {
       y.z += in ? yp[j].z : 0.f; y.w += in ? yp[j].w : 0.f;
     }
   }
+  constexpr float kBack = 1.f / kFactorScale;
+  y.x *= kBack; y.y *= kBack; y.z *= kBack; y.w *= kBack;
   float4 v = y;
   if (!a.first_slice) {
     v.x = o.x * al + y.x; v.y = o.y * al + y.y; v.z = o.z * al + y.z; v.w = o.w * al + y.w;

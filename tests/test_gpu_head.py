@@ -164,6 +164,52 @@ def test_head_steps_of_many_slices(n):
     np.testing.assert_array_equal(out["best_idx"].cpu().numpy(), res["best_idx"])
 
 
+@pytest.mark.parametrize("one_step", [True, False])
+@pytest.mark.parametrize("where", ["first", "last"])
+def test_head_gradient_of_confident_rows(where, one_step):
+    """Rows that give their target, in the vocabulary's first or last slice, 18 more than the other
+    logits' standard deviation of 1.5, with weight rows around a common mean: dH is the sum of
+    151935 small weights times their rows. Every logit is exact in fp16 (multiples of 1/64 below 32).
+    The bound, per element: fp16's rounding of dH, of P, of the tile's factor and of their product
+    (2^-11 each, of the sum of p |w|); P's subnormals in the target's own tile (2^-25 each); the fp32
+    sums, whose rounding errors (2^-24 of a partial sum of at most |w[target]|, one per MFMA step
+    and part) add up at random."""
+    _case(f"head confident rows, target in the {where} slice, one step: {one_step}")
+    rng = np.random.default_rng(14)
+    vocab, hidden, n, vchunk = 151936, 64, 6, 8192
+    h = np.stack([rng.permutation(np.repeat([1.0, -1.0], hidden // 2)) for _ in range(n)])
+    w = 0.25 + np.rint(rng.standard_normal((vocab, hidden)) * 12) / 64
+    t = np.arange(n) * 37 + (100 if where == "first" else vocab - 1000)
+    w[t] += h * (18 / 64)
+    h, w = h.astype(np.float16), w.astype(np.float16)
+    ref = head_oracle.head_direct(h, w, t)
+    z = head_oracle.logits16(h, w).astype(np.float64)
+    assert np.array_equal(z, h.astype(np.float64) @ w.astype(np.float64).T)
+    dev = [torch.from_numpy(x).to(DEV) for x in (h, w, t)]
+    if one_step:
+        got = fused_head.head_ce(*dev, vocab_chunk=vchunk, n_grad=n)["grad"]
+    else:  # a workspace of `group` slices a step
+        group = fused_head.GROUP
+        ws = torch.empty(_ops.head_ce_workspace_bytes(n, hidden, group * vchunk, vchunk, n, group),
+                         dtype=torch.uint8, device=DEV)
+        f32 = [torch.empty(n, device=DEV) for _ in range(2)]
+        i32 = [torch.empty(n, dtype=torch.int32, device=DEV) for _ in range(2)]
+        got = torch.empty_like(dev[0])
+        torch.ops.talm.head_ce(*dev, vchunk, n, group, *f32, *i32, got, ws)
+    p = np.exp(z - z.max(1)[:, None])
+    p /= p.sum(1)[:, None]
+    p[np.arange(n), t] = 0
+    absw = np.abs(w.astype(np.float64))
+    steps = vocab / 16 + 48
+    bound = (2.0 ** -11 * np.abs(ref["grad"]) + 2.0 ** -25 + 3 * 2.0 ** -11 * (p @ absw)
+             + 127 * 2.0 ** -25 * absw.max() + 4 * np.sqrt(steps) * 2.0 ** -24 * absw[t])
+    err = np.abs(got.double().cpu().numpy() - ref["grad"])
+    rel = np.linalg.norm(err, axis=1) / np.linalg.norm(ref["grad"], axis=1)
+    print(f"[head] p {1 - p.sum(1).max():.4f}, relative error of dH {rel.max():.2e}, "
+          f"of the bound {(err / bound).max():.2f}", flush=True)
+    assert np.all(err <= bound)
+
+
 @pytest.mark.parametrize("n_grad", [0, 70])
 def test_head_workspace_of_the_smaller_step(n_grad):
     """A workspace that holds `group` slices a step but not more (one kept from another call) still
