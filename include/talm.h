@@ -219,7 +219,7 @@ int talm_swiglu_bwd_rows(const uint16_t* grad, int64_t ld_grad, const uint16_t* 
 /*
  * Bytes of workspace talm_head_ce needs (-1 for arguments it would reject). At least
  * `group` vocabulary slices are processed per step, more where few rows leave room (the gradient
- * rows' e^{z - m} within 168 MiB; without gradient rows, the statistics within 64 MiB): the workspace
+ * rows' e^{z - m} within 168 MiB and every row's statistics within 64 MiB): the workspace
  * holds a step's fp16 e^{z - m} [n_grad, slices * vchunk], its per-tile statistics and the fp32
  * gradient partials [parts, n_grad, hidden].
  */

@@ -935,22 +935,24 @@ GradPlan plan_grad(int64_t n_grad, int64_t hidden, int64_t group_cols) {
 }
 
 // Slices per step of the slice loop (a step is one launch each of head_logits, head_merge,
-// head_grad and head_combine): at least `group`, and as many more as fit the bound of what a step
+// head_grad and head_combine): at least `group`, and as many more as fit the bounds of what a step
 // leaves behind.
-// - With gradient rows that is P (2 bytes per gradient row and column), written by head_logits and
+// - The tiles' statistics (16 bytes per row and 128 columns), of every row, labelled or not: 64 MiB
+//   (3500 rows at a vocabulary of 151936; evaluation, five slices a step / so: 64 rows 259 / 166 us, 517
+//   400 / 328, 1167 733 / 590, 2048 984 / 963).
+// - P of the gradient rows (2 bytes per gradient row and column), written by head_logits and
 //   read by head_grad: 168 MiB of it stay in the 256 MiB last-level cache beside the weights. Fewer,
 //   larger launches fill the chip better (hidden 1536, vocabulary 151936, training, against five
 //   slices a step: 64 rows 514 -> 293 us, 257 681 -> 483, 517 805 -> 705, 1167 1390 -> 1285; at
 //   1843 and 2048 rows eight slices, 241 and 268 MB of P, cost 4% and 7%).
-// - Without, only the tiles' statistics (16 bytes per row and 128 columns): 64 MiB (3500 rows at a
-//   vocabulary of 151936; 64 rows 259 -> 166 us, 517 400 -> 328, 1167 733 -> 590, 2048 984 -> 963).
+constexpr int64_t kStepStats = int64_t{64} << 20, kStepP = int64_t{168} << 20;
+
 int slices_per_step(int64_t n_rows, int64_t vocab, int64_t vchunk, int64_t n_grad, int group) {
   const int64_t slices = (vocab + vchunk - 1) / vchunk;
-  const int64_t per_slice = n_grad > 0 ? n_grad * vchunk * 2 : n_rows * (vchunk / kTile) * 16;
-  const int64_t bound = int64_t{n_grad > 0 ? 168 : 64} << 20;
-  const int64_t most = std::min(
-      slices, std::max<int64_t>(group, std::min(bound / std::max<int64_t>(per_slice, 1),
-                                                ((int64_t{1} << 22) - 1) / vchunk)));
+  const int64_t fit = std::min({kStepStats / std::max<int64_t>(n_rows * (vchunk / kTile) * 16, 1),
+                                kStepP / std::max<int64_t>(n_grad * vchunk * 2, 1),
+                                ((int64_t{1} << 22) - 1) / vchunk});
+  const int64_t most = std::min(slices, std::max<int64_t>(group, fit));
   const int64_t steps = (slices + most - 1) / most;  // of nearly equal size: 19 slices go 10 + 9
   return static_cast<int>(std::min(slices, std::max<int64_t>(group, (slices + steps - 1) / steps)));
 }

@@ -12,7 +12,8 @@ On MI355X the whole slice loop is ONE call of talm_head_ce (talm_amd/csrc/head_c
 GEMMs are hand-written fp16 MFMA kernels whose epilogue / prologue do the statistics and the
 e^{z - m} weights, so a slice's logits are written once (fp16) and read once, and the per-slice
 accumulator GEMM, which the reference leaves to cuBLAS, runs once per group of slices
-(`GROUP` of them, or as many more as keep the rows' weights within 168 MiB):
+(`GROUP` of them, or as many more as keep the labelled rows' weights within 168 MiB and every row's
+statistics within 64 MiB):
 the reference's per-slice rescales of the accumulator telescope over a group, so the group's
 columns form one reduction, cut into as many K parts as fill the chip (fp32 partials summed in
 part order, then one rescale of the accumulator per group).

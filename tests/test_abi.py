@@ -63,6 +63,18 @@ def test_argument_rejection_needs_no_gpu():
     assert status == _lib.TALM_EINVAL and b"256-byte" in lib.talm_last_error()
 
 
+@pytest.mark.parametrize("rows,n_grad", [(517, 0), (4096, 400), (16384, 200), (65536, 400),
+                                         (131072, 500), (131072, 0), (2048, 1843)])
+def test_head_workspace_is_bounded_over_the_group_of_slices(rows, n_grad):
+    """Steps of more than `group` slices add at most 64 MiB of statistics (of every row, labelled
+    or not), 168 MiB of P and 64 MiB of partials (256 workgroups' 256 x 256 fp32 tiles)."""
+    size = _lib.lib().talm_head_ce_workspace
+    group = 5
+    few = size(rows, 1536, group * 8192, 8192, n_grad, group)
+    extra = 64 + (168 + 64 if n_grad else 0)
+    assert size(rows, 1536, 151936, 8192, n_grad, group) <= few + (extra << 20)
+
+
 def test_custom_ops_are_registered_for_the_gpu_only():
     import torch
 
