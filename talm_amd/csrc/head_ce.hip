@@ -515,13 +515,15 @@ __device__ __forceinline__ int lanes_min(int v) {
 }
 
 // The lanes' statistics as one: the maximum first, then each lane's sums rescaled to it once and
-// added; the first argmax among the lanes that hold the maximum.
+// added; the first argmax among the lanes that hold the maximum. A lane without a finite logit (its
+// tile past the slice, or overflowed to -inf throughout, with sums of NaN then) adds nothing: a
+// select, as NaN times 0 is NaN.
 __device__ __forceinline__ Stat lanes_stat(Stat v) {
   Stat r;
   r.m = lanes_max(v.m);
-  const float e = v.m == -INFINITY ? 0.f : __expf(v.m - r.m);
-  r.s = lanes_sum(v.s * e);
-  r.t = lanes_sum(v.t * e);
+  const float e = __expf(v.m - r.m);
+  r.s = lanes_sum(v.m == -INFINITY ? 0.f : v.s * e);
+  r.t = lanes_sum(v.m == -INFINITY ? 0.f : v.t * e);
   r.idx = lanes_min(v.m == r.m ? v.idx : 0x7fffffff);
   return r;
 }

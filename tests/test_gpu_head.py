@@ -164,6 +164,29 @@ def test_head_steps_of_many_slices(n):
     np.testing.assert_array_equal(out["best_idx"].cpu().numpy(), res["best_idx"])
 
 
+@pytest.mark.parametrize("vchunk", [1024, 16384])  # a tile per lane, and lane-strided loops
+def test_head_tile_that_overflows_to_minus_infinity(vchunk):
+    """Logits that all overflow fp16 to -inf in one statistics tile of 128 columns have probability
+    0: losses, entropies and argmax are those of the vocabulary without them."""
+    _case(f"head tile of -inf, vchunk={vchunk}")
+    h16, w16, t = exact_head_case(40, 64, 9000, 21)
+    h16[:, 0] = 256.0
+    w16[:, 0] = 0.0
+    gone = np.arange(9000) // 128 == 37
+    w16[gone] = 0.0
+    w16[gone, 0] = -512.0  # -131072
+    t[gone[np.maximum(t, 0)] & (t >= 0)] = 5
+    out = fused_head.head_ce(*(torch.from_numpy(x).to(DEV) for x in (h16, w16, t)),
+                             vocab_chunk=vchunk, need_grad=False)
+    kept = np.flatnonzero(~gone)
+    place = np.cumsum(~gone) - 1
+    ref = head_oracle.head_direct(h16, w16[kept], np.where(t >= 0, place[np.maximum(t, 0)], t))
+    got = {k: v.cpu().numpy() for k, v in out.items() if v is not None}
+    assert np.all(np.abs(got["token_loss"] - ref["token_loss"]) <= 2e-5 + 2e-6 * ref["zmax"])
+    assert np.all(np.abs(got["entropy"] - ref["entropy"]) <= 2e-5 + 1e-5 * ref["zmax"])
+    assert np.array_equal(got["best_idx"], kept[ref["best_idx"]])
+
+
 @pytest.mark.parametrize("one_step", [True, False])
 @pytest.mark.parametrize("where", ["first", "last"])
 def test_head_gradient_of_confident_rows(where, one_step):
