@@ -169,6 +169,8 @@ def labelled_first(labelled, n_labelled):
 
 def _order_rows(h16, targets, n_labelled):
     """(hidden rows, targets) in `labelled_first`'s order and its dest, in one launch."""
+    if h16.stride(0) < h16.shape[1]:  # expanded or overlapping rows
+        h16 = h16.contiguous()
     out = torch.empty(h16.shape, dtype=torch.float16, device=h16.device)
     rows_targets, dest = torch.empty_like(targets), torch.empty_like(targets)
     torch.ops.talm.head_order(h16, targets, n_labelled, out, rows_targets, dest)

@@ -112,6 +112,26 @@ def test_head_every_row_a_gradient_row(labels):
     _check(res, h16, w16, t, 1024, what=f"all rows {labels}")
 
 
+@pytest.mark.parametrize("stride", [0, 8])
+def test_head_orders_overlapping_rows(stride):
+    """Hidden rows that share memory (an expanded row, stride 0, or rows 8 columns apart) with
+    some labels ignored: the same as of a contiguous copy, bit for bit."""
+    _case(f"head overlapping rows, stride {stride}")
+    h16, w16, t = exact_head_case(37, 64, 1000, 22)
+    base = torch.from_numpy(h16).to(DEV).flatten()
+    rows = base.as_strided((37, 64), (stride, 1))
+    assert 0 < int((t >= 0).sum()) < 37
+    outs = []
+    for x in (rows.contiguous(), rows):
+        x = x.detach().requires_grad_()
+        loss, *per_row = fused_head.fused_head_loss(x, torch.from_numpy(w16).to(DEV),
+                                                    torch.from_numpy(t).to(DEV), None, 256)
+        loss.backward()
+        outs.append([loss.detach(), *per_row, x.grad])
+    for a, b in zip(*outs):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("num_items", [None, 7, "tensor"])
 def test_head_num_items_denominator(num_items):
     _case(f"head num_items={num_items}")
