@@ -573,12 +573,15 @@ int talm_nf4_gemm_partials(const uint16_t* x, int64_t ldx, int64_t n_tokens, con
  *
  * talm_head_order: the rows of hidden f16 [n, hidden] (row stride ldh, a multiple of 8; hidden too)
  * and their targets in labelled-first order: row r to dest[r] = the number of labelled rows before
- * it (target >= 0), or n_labelled + the unlabelled rows before it; n_labelled is the exact count.
+ * it (target >= 0), or n_labelled + the unlabelled rows before it; n_labelled is the exact count (with
+ * another one, the rows left without a place get dest -1, and rows of out that none goes to are not
+ * written).
  * out f16 [n, hidden] contiguous, targets_out, dest i64 [n]. Replaces solution/fused_head.py:290-299
  * with the two gathers of :328-336.
  *
  * talm_head_restore: row r of each output is row dest[r] of its input (token_loss, entropy f32,
- * correct, best_idx i32 [n], grad f16 [n, hidden] contiguous). Replaces the gathers back to the
+ * correct, best_idx i32 [n], grad f16 [n, hidden] contiguous); where dest[r] is outside [0, n), NaN
+ * (correct 0, best_idx -1). Replaces the gathers back to the
  * input order (solution/fused_head.py:374-383).
  *
  * talm_scale_rows: out[i] = fp16(fp32(g[i]) * s), s = *grad_loss / *denom (0 when *denom is 0),

@@ -174,6 +174,9 @@ __global__ __launch_bounds__(kBlock) void scatter_rows_kernel(
 // launches of 2-5 us on the GPU and about 10 us each on the host (a mask, an arange, a cumulative
 // sum, the selects and gathers). With the restore below: head and its gradient at 2048 rows 2096 ->
 // 2060 us, a two-layer training step on a slow host 3816 -> 3578.
+// Where n_labelled is not the rows' own count, the rows that have no place of their own (a labelled
+// row past n_labelled, an unlabelled one past the last row) get dest -1 and go nowhere, which the
+// restore below turns into NaN: such a call must not pass for a right one.
 __global__ __launch_bounds__(256) void head_order_kernel(
     const uint16_t* __restrict__ hidden, int64_t ldh, const int64_t* __restrict__ targets,
     int64_t n, int64_t n_labelled, int cols8, int rows, uint16_t* __restrict__ out,
@@ -194,15 +197,15 @@ __global__ __launch_bounds__(256) void head_order_kernel(
     const uint64_t mask = __ballot(t >= 0);
     const int64_t before = seen + __popcll(mask & ((uint64_t{1} << lane) - 1));
     const int64_t to = t >= 0 ? before : n_labelled + row - before;
-    // a count that is not the rows' own must not place a row outside the buffers
-    const int64_t at = min(max(to, int64_t{0}), n - 1);
+    const int64_t at = to < (t >= 0 ? n_labelled : n) ? to : -1;
     if (wave == 0 && row < end) {
       dest[row] = at;
-      targets_out[at] = t;
+      if (at >= 0) targets_out[at] = t;
     }
     const int here = static_cast<int>(min(end - r, int64_t{kWave}));
     for (int k = wave; k < here; k += 256 / kWave) {
       const int64_t to_k = __shfl(at, k, kWave);
+      if (to_k < 0) continue;
       const uint4* src = reinterpret_cast<const uint4*>(hidden + (r + k) * ldh);
       uint4* dst = reinterpret_cast<uint4*>(out) + to_k * cols8;
       for (int c = lane; c < cols8; c += kWave) dst[c] = src[c];
@@ -212,7 +215,8 @@ __global__ __launch_bounds__(256) void head_order_kernel(
 }
 
 // The head's per-row outputs and gradient back to the input order: row r takes row dest[r] of each,
-// one wavefront per row (one launch for five gathers).
+// one wavefront per row (one launch for five gathers). A row without a place (dest[r] outside
+// [0, n)) gets NaN, no prediction (-1) and not correct.
 struct HeadRows {
   const float* token_loss;
   const float* entropy;
@@ -233,9 +237,19 @@ __global__ __launch_bounds__(256) void head_restore_kernel(HeadRows in, HeadRows
   const int lane = threadIdx.x & 63;
   const int64_t row = static_cast<int64_t>(blockIdx.x) * (256 / kWave) + (threadIdx.x >> 6);
   if (row >= n) return;
-  const int64_t at = min(max(dest[row], int64_t{0}), n - 1);
-  const uint4* src = reinterpret_cast<const uint4*>(in.grad) + at * cols8;
+  const int64_t at = dest[row];
   uint4* dst = reinterpret_cast<uint4*>(out.grad) + row * cols8;
+  if (at < 0 || at >= n) {
+    constexpr uint32_t kNan2 = 0x7e007e00u;  // two fp16 NaN
+    for (int c = lane; c < cols8; c += kWave) dst[c] = make_uint4(kNan2, kNan2, kNan2, kNan2);
+    if (lane == 0) {
+      out.token_loss[row] = out.entropy[row] = __builtin_nanf("");
+      out.correct[row] = 0;
+      out.best_idx[row] = -1;
+    }
+    return;
+  }
+  const uint4* src = reinterpret_cast<const uint4*>(in.grad) + at * cols8;
   for (int c = lane; c < cols8; c += kWave) dst[c] = src[c];
   if (lane == 0) {
     out.token_loss[row] = in.token_loss[at];

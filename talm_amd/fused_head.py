@@ -239,7 +239,8 @@ def fused_head_loss(hidden, weight, targets, num_items=None, vocab_chunk=None, *
     shifted (-100 = ignore). Returns (loss, token_loss[N], token_entropy[N], correct[N]) and, with
     `return_argmax`, the per-token argmax [N] (int32) as a fifth element
     (solution/fused_head.py:447-462). `n_labelled`: the exact host count of targets >= 0 when the
-    caller has it (saves a host sync). `grad_all_rows`: every row is a gradient row (no
+    caller has it (saves a host sync; with a gradient, a wrong count strictly between 0 and N makes
+    the loss NaN). `grad_all_rows`: every row is a gradient row (no
     labelled-first reordering, no count; an ignored row's gradient is zero), so no launch depends
     on a host value of the targets (a step captured in a HIP graph). `token_chunk` (the
     reference's token-chunked path) runs the same kernel `token_chunk` rows at a time."""

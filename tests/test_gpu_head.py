@@ -132,6 +132,30 @@ def test_head_orders_overlapping_rows(stride):
         assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("off", [-3, 2])
+def test_head_wrong_label_count_is_not_silent(off):
+    """A label count that is not the targets' own leaves rows without a place in the labelled-first
+    order: the loss and those rows' outputs and gradients are NaN, the other rows' are right."""
+    _case(f"head label count off by {off}")
+    h16, w16, t = exact_head_case(300, 64, 1000, 23)
+    count = int((t >= 0).sum())
+    x = torch.from_numpy(h16).to(DEV).requires_grad_()
+    w, tt = torch.from_numpy(w16).to(DEV), torch.from_numpy(t).to(DEV)
+    ref = fused_head.fused_head_loss(x, w, tt, 1.0, 256, n_labelled=count, return_argmax=True)
+    (ref_grad,) = torch.autograd.grad(ref[0], x)
+    got = fused_head.fused_head_loss(x, w, tt, 1.0, 256, n_labelled=count + off, return_argmax=True)
+    (grad,) = torch.autograd.grad(got[0], x)
+    assert got[0].isnan()
+    # the last labelled rows past the count, or the last unlabelled rows past the end
+    lost = (tt >= 0).nonzero().flatten()[off:] if off < 0 else (tt < 0).nonzero().flatten()[-off:]
+    kept = torch.ones(300, dtype=torch.bool, device=DEV)
+    kept[lost] = False
+    assert got[1][lost].isnan().all() and got[2][lost].isnan().all() and grad[lost].isnan().all()
+    assert not got[3][lost].any() and (got[4][lost] == -1).all()
+    for a, b in zip((*got[1:], grad), (*ref[1:], ref_grad)):
+        assert torch.equal(a[kept], b[kept])
+
+
 @pytest.mark.parametrize("num_items", [None, 7, "tensor"])
 def test_head_num_items_denominator(num_items):
     _case(f"head num_items={num_items}")
