@@ -805,10 +805,12 @@ void launch_proj(QkvArgs& a, hipStream_t stream) {
   a.cs_vec = a.cos && aligned(a.cos, 16) && aligned(a.sin, 16) && a.cs_stride % 4 == 0;
   // 128-row tiles once the 64-row ones exceed one round at two workgroups per CU. Measured, 64 / 128
   // rows: forward at 3000 tokens 46.5 / 36.6 us, at 5015 73.0 / 68.8, input gradient 41.3 / 31.9 and 54.7 /
-  // 39.2; at 2048 tokens and below (one round of 64-row tiles) half as many workgroups would run.
+  // 39.2; at 2048 tokens and below (one round of 64-row tiles) half as many workgroups would run. A
+  // tile's rows of x and of the extra step's operand must lie within 32-bit offsets.
   const int64_t small = static_cast<int64_t>((a.n_tokens + QkvShape::kBM - 1) / QkvShape::kBM) *
                         ((a.n_out + QkvShape::kBN - 1) / QkvShape::kBN);
-  if (small > 2 * device_cus() && fits32(QkvWide::kBM, a.ldx))
+  if (small > 2 * device_cus() && fits32(QkvWide::kBM, a.ldx) &&
+      (kDown || fits32(QkvWide::kBM, a.ldt)))
     launch_tiles<QkvWide, kDown>(a, stream);
   else
     launch_tiles<QkvShape, kDown>(a, stream);

@@ -173,6 +173,23 @@ def test_projections_on_128_row_tiles(n):
     test_qkv_lora_bwd_dx_matches_fp32(n, 2048, 256, 32)
 
 
+def test_extra_step_with_a_wide_row_stride():
+    """128 rows of u 2^23 + 2^17 columns apart: 64-row tiles reach them with 32-bit offsets, 128-row
+    ones would not (516 tiles of 64 x 128, more than a round). The same bits as of contiguous rows."""
+    n, k, size, rank = 128, 64, 258 * 128, 8
+    _case(f"projection, wide rows of u: {n} x {k} -> {size}")
+    g = torch.Generator().manual_seed(6)
+    dcat, wt, u, at = (torch.randn(*s, generator=g).half().to(DEV)
+                       for s in ((n, k), (size, k), (n, rank), (size, rank)))
+    wide = torch.empty(n, 2 ** 23 + 2 ** 17, dtype=torch.float16, device=DEV)[:, :rank]
+    wide.copy_(u)
+    outs = []
+    for rows in (u, wide):
+        outs.append(torch.empty(n, size, dtype=torch.float16, device=DEV))
+        torch.ops.talm.qkv_lora_bwd_dx(dcat, wt, rows, at, outs[-1])
+    assert torch.equal(*outs)
+
+
 def test_rotation_with_unaligned_tables():
     """cos / sin rows that are not 16-byte aligned (row stride 129) rotate to the same bits."""
     n, size, n_out = 77, 64, 384
