@@ -63,6 +63,22 @@ def _check(res, h16, w16, t, vchunk, num_items=None, grad_scale=3.0, exact=True,
     return ref
 
 
+def _head_ce_by_group(h, w, t, vchunk, n_grad, group):
+    """talm_head_ce with a workspace that holds `group` slices a step and no more (for inputs
+    where a step would take more): as fused_head.head_ce returns it."""
+    n, hidden = h.shape
+    vocab = w.shape[0]
+    size = _ops.head_ce_workspace_bytes(n, hidden, group * vchunk, vchunk, n_grad, group)
+    assert size < _ops.head_ce_workspace_bytes(n, hidden, vocab, vchunk, n_grad, group)
+    out = {k: torch.empty(n, dtype=d, device=DEV) for k, d in
+           (("token_loss", torch.float32), ("entropy", torch.float32),
+            ("best_idx", torch.int32), ("correct", torch.int32))}
+    out["grad"] = torch.empty_like(h) if n_grad else None
+    ws = torch.empty(size, dtype=torch.uint8, device=DEV)
+    torch.ops.talm.head_ce(h, w, t, vchunk, n_grad, group, *out.values(), ws)
+    return out
+
+
 @pytest.mark.parametrize("n,hidden,vocab,vchunk,seed", [
     (37, 64, 4097, 4096, 1), (300, 256, 1000, 384, 2), (5, 1536, 151936, 8192, 3),
     (2, 16, 5, 128, 4), (129, 32, 20000, 8192, 5), (64, 8, 1, 128, 6)])
@@ -169,7 +185,8 @@ def test_head_num_items_denominator(num_items):
 
 def test_head_argmax_ties_across_slices_and_groups():
     """solution/test_kernels.py:250-282 at full width: two equal largest logits (exactly 64)
-    inside one tile, across tiles, across slices and across slice groups: the first wins."""
+    inside one tile, across tiles, across slices and, in steps of GROUP slices (which so few rows
+    take only with a workspace for no more), across steps: the first wins."""
     _case("head ties")
     rng = np.random.default_rng(13)
     vocab, hidden = 151936, 256
@@ -186,8 +203,53 @@ def test_head_argmax_ties_across_slices_and_groups():
         h[2 * i] = h[2 * i + 1] = (signs * 4).astype(np.float16)
         t[2 * i], t[2 * i + 1] = a, b
     res = _run(h, w, t, vchunk=8192)
-    assert res["correct"][:2 * len(pairs)].tolist() == [True, False] * len(pairs)
-    assert res["best_idx"][:2 * len(pairs)].tolist() == [a for a, _ in pairs for _ in range(2)]
+    dev = [torch.from_numpy(x).to(DEV) for x in (h, w, t)]
+    stepped = _head_ce_by_group(*dev, 8192, len(h), fused_head.GROUP)
+    for r in (res, {k: v.cpu().numpy() for k, v in stepped.items()}):
+        assert r["correct"][:2 * len(pairs)].tolist() == [True, False] * len(pairs)
+        assert r["best_idx"][:2 * len(pairs)].tolist() == [a for a, _ in pairs for _ in range(2)]
+
+
+def test_head_two_steps_of_more_than_eight_slices():
+    """700 gradient rows at full width take steps of ten and nine slices: a second set of a step's
+    statistics on top of stored ones, and an accumulator rescaled once. Every seventeenth row
+    against the oracle, all of them against steps of GROUP slices."""
+    _case("head steps of 10 and 9 slices")
+    n, vocab, vchunk = 700, 151936, 8192
+    h16, w16, t = exact_head_case(n, 64, vocab, 24)
+    t = np.where(t >= 0, t, 7)
+    dev = [torch.from_numpy(x).to(DEV) for x in (h16, w16, t)]
+    out = fused_head.head_ce(*dev, vchunk, n)
+    stepped = _head_ce_by_group(*dev, vchunk, n, fused_head.GROUP)
+    for k in ("best_idx", "correct"):
+        assert torch.equal(out[k], stepped[k])
+    rows = np.arange(0, n, 17)
+    ref = head_oracle.head_direct(h16[rows], w16, t[rows])
+    scale = np.abs(ref["grad"]).max(1, keepdims=True)
+    for res in (out, stepped):
+        got = {k: v.cpu().numpy()[rows] for k, v in res.items()}
+        assert np.all(np.abs(got["token_loss"] - ref["token_loss"]) <= 2e-5 + 2e-6 * ref["zmax"])
+        assert np.all(np.abs(got["entropy"] - ref["entropy"]) <= 2e-5 + 1e-5 * ref["zmax"])
+        assert np.array_equal(got["best_idx"], ref["best_idx"])
+        assert np.all(np.abs(got["grad"] - ref["grad"]) <= 2e-3 * np.abs(ref["grad"]) + 2.0 ** -7 * scale)
+
+
+@pytest.mark.parametrize("group", [None, 1])
+def test_head_slices_wider_than_a_tile_per_lane(group):
+    """Slices of more than 64 tiles (here 128, and a last one of 57): their statistics are taken in
+    lane-strided loops, all slices in one step or one a step; rows past two 128-row blocks, some
+    of them without a gradient."""
+    _case(f"head wide slices, group {group}")
+    n, n_grad, vocab, vchunk = 300, 270, 40000, 16384
+    h16, w16, t = exact_head_case(n, 64, vocab, 25)
+    t[n_grad:] = -100
+    dev = [torch.from_numpy(x).to(DEV) for x in (h16, w16, t)]
+    out = (fused_head.head_ce(*dev, vchunk, n_grad) if group is None
+           else _head_ce_by_group(*dev, vchunk, n_grad, group))
+    res = {k: v.float().cpu().numpy() if k == "grad" else v.cpu().numpy() for k, v in out.items()}
+    n_lab = int((t >= 0).sum())
+    res["loss"] = res["token_loss"].astype(np.float64).sum() / n_lab
+    _check(res, h16, w16, t, vchunk, grad_scale=n_lab, what=f"group {group}")
 
 
 @pytest.mark.parametrize("n", [1, 192, 193, 256, 257, 450])
@@ -255,14 +317,8 @@ def test_head_gradient_of_confident_rows(where, one_step):
     dev = [torch.from_numpy(x).to(DEV) for x in (h, w, t)]
     if one_step:
         got = fused_head.head_ce(*dev, vocab_chunk=vchunk, n_grad=n)["grad"]
-    else:  # a workspace of `group` slices a step
-        group = fused_head.GROUP
-        ws = torch.empty(_ops.head_ce_workspace_bytes(n, hidden, group * vchunk, vchunk, n, group),
-                         dtype=torch.uint8, device=DEV)
-        f32 = [torch.empty(n, device=DEV) for _ in range(2)]
-        i32 = [torch.empty(n, dtype=torch.int32, device=DEV) for _ in range(2)]
-        got = torch.empty_like(dev[0])
-        torch.ops.talm.head_ce(*dev, vchunk, n, group, *f32, *i32, got, ws)
+    else:
+        got = _head_ce_by_group(*dev, vchunk, n, fused_head.GROUP)["grad"]
     p = np.exp(z - z.max(1)[:, None])
     p /= p.sum(1)[:, None]
     p[np.arange(n), t] = 0
@@ -285,13 +341,8 @@ def test_head_workspace_of_the_smaller_step(n_grad):
     group, vchunk, vocab = 3, 128, 9 * 128
     h16, w16, t = exact_head_case(70, 64, vocab, 50)
     h, w, tt = [torch.from_numpy(x).to(DEV) for x in (h16, w16, t)]
-    small = _ops.head_ce_workspace_bytes(70, 64, group * vchunk, vchunk, n_grad, group)
-    assert small < _ops.head_ce_workspace_bytes(70, 64, vocab, vchunk, n_grad, group)
     full = fused_head.head_ce(h, w, tt, vchunk, n_grad, n_grad > 0, group)
-    got = {k: torch.empty_like(v) for k, v in full.items() if v is not None}
-    ws = torch.empty(small, dtype=torch.uint8, device=DEV)
-    torch.ops.talm.head_ce(h, w, tt, vchunk, n_grad, group, got["token_loss"], got["entropy"],
-                           got["best_idx"], got["correct"], got.get("grad"), ws)
+    got = _head_ce_by_group(h, w, tt, vchunk, n_grad, group)
     assert torch.equal(got["best_idx"], full["best_idx"])
     assert torch.equal(got["token_loss"], full["token_loss"])
     if n_grad:  # one fp16 rounding of each column's factor, one of dH
