@@ -28,7 +28,7 @@ ARCH = "gfx950"
 # v_pk_{add,mul,fma}_f32); hipcc's host pass warns that it does not know the feature.
 DEVICE_FLAGS = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 COMMON_FLAGS = [f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC", "-fvisibility=hidden",
-                "-Wall", "-Wno-unused-function"]
+                "-Wall"]
 
 
 def hipcc():

@@ -9,9 +9,10 @@
 //
 // The forward is a flash-attention pass per (sequence, query tile, query heads of one KV head),
 // 32 query rows of a head per wavefront, its key tiles of 64 streamed with direct-to-LDS loads and,
-// where few workgroups leave the chip idle, split between two groups of wavefronts. Scores are computed transposed, S^T = K Q^T (v_mfma_f32_32x32x16_f16), so
-// each lane owns one query row (its accumulator column): the online max / sum and the output
-// rescale are per-lane scalars. The exponentiated scores are already in the B-operand layout of
+// where few workgroups leave the chip idle, split between two groups of wavefronts. Scores are
+// computed transposed, S^T = K Q^T (v_mfma_f32_32x32x16_f16), so each lane owns one query row (its
+// accumulator column): the online max / sum and the output rescale are per-lane scalars. The
+// exponentiated scores are already in the B-operand layout of
 // O^T = V^T P^T: the reduction over keys takes the accumulator's key order as its k-slot order,
 // and V^T is read in that same order from the row-major V tile with transposing LDS reads. The
 // row statistics are kept in base 2 (scores times scale * log2 e); lse is written in natural-log
@@ -93,40 +94,27 @@ constexpr int kTileBytes = kKeys * kD * 2;  // 16 KiB
 __device__ __forceinline__ int tile_swz(int row) { return ((row & 3) << 2) | ((row >> 2) & 3); }
 __device__ __forceinline__ int tile_chunk(int row, int chunk) { return row * 16 + (chunk ^ tile_swz(row)); }
 
+__device__ __forceinline__ uint32_t lds_addr(const unsigned char* lds) {
+  return static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
+      (__attribute__((address_space(3))) const unsigned char*)(lds)));
+}
+
+// LDS reads at an address plus a constant offset, as inline assembly. The compiler does not track
+// them: it adds no wait for the direct-to-LDS loads in flight before them (it cannot tell that
+// those write the other ring slot, and would wait for all of them), and the caller waits for the
+// results itself (lgkm_wait, lgkm_wait8) before using them.
+//
 // ds_read_b64_tr_b16 (gfx950): within each 16-lane group, lane i receives element e (0..3) from
 // row 4 e + i / 4 of the 16 x 4 matrix formed by the four halves at each lane's address, column
 // i % 4 (checked on the GPU with an in-bounds probe). With lane j pointing at row K0 + j / 4,
 // columns D0 + 4 (j % 4) of a row-major [keys][d] tile, lane i gets keys K0 .. K0 + 3 of column
 // D0 + i: the transpose of 4 x 16 elements.
-// A 32 x 16 operand of v_mfma_f32_32x32x16_f16 read transposed from a swizzled [rows][128]
-// tile: A[m][k] = tile[row0 + key(k)][col0 + m], lane l holding m = l % 32 and k-slots
-// 8 (l / 32) .. + 7, whose rows follow the accumulator order of the 32-row blocks: slots
-// 8 hh + e hold rows row0 + 4 hh + e (e < 4) and row0 + 8 + 4 hh + e - 4 (e >= 4).
-// The same operand's two halves issued as inline assembly. The compiler does not track these
-// reads: it adds no wait for the direct-to-LDS loads in flight before them (it cannot tell that
-// those write the other ring slot, and would wait for all of them), and the caller waits for the
-// results itself with lgkm_wait8 before using them.
-__device__ __forceinline__ half4_t read_tr_untracked(const unsigned char* lds) {
-  const uint32_t addr = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
-      (__attribute__((address_space(3))) const unsigned char*)(lds)));
-  half4_t r;
-  asm volatile("ds_read_b64_tr_b16 %0, %1" : "=v"(r) : "v"(addr));
-  return r;
-}
-__device__ __forceinline__ void read_tr_operand_untracked(const unsigned char* tile, int row0,
-                                                          int col0, int lane, half4_t& lo,
-                                                          half4_t& hi) {
-  const int g = lane >> 4, i = lane & 15, hh = g >> 1;
-  const int col = col0 + 16 * (g & 1) + 4 * (i & 3);
-  const int row = row0 + 4 * hh + (i >> 2);
-  lo = read_tr_untracked(tile + tile_chunk(row, col >> 3) * 16 + (col & 7) * 2);
-  hi = read_tr_untracked(tile + tile_chunk(row + 8, col >> 3) * 16 + (col & 7) * 2);
-}
-// The same at an LDS address plus a constant offset, and a 16-byte read likewise.
-__device__ __forceinline__ uint32_t lds_addr(const unsigned char* lds) {
-  return static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
-      (__attribute__((address_space(3))) const unsigned char*)(lds)));
-}
+// Two of them make a 32 x 16 operand of v_mfma_f32_32x32x16_f16 transposed from a swizzled
+// [rows][128] tile: A[m][k] = tile[row0 + key(k)][col0 + m], lane l holding m = l % 32 and k-slots
+// 8 hh .. + 7 (hh = l / 32), whose rows follow the accumulator order of the 32-row blocks: slots
+// 8 hh + e hold rows row0 + 4 hh + e (e < 4, the first read) and row0 + 8 + 4 hh + e - 4 (e >= 4, the
+// second, 8 rows on). With g = l / 16 and i = l % 16 the lane points at row row0 + 4 hh + i / 4,
+// columns col0 + 16 (g % 2) + 4 (i % 4) .. + 3.
 __device__ __forceinline__ half4_t read_tr_untracked(uint32_t addr, int off) {
   half4_t r;
   asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(r) : "v"(addr), "n"(off));
@@ -158,16 +146,6 @@ __device__ __forceinline__ void lgkm_wait(int n, half8_t& r, half8_t& q) {
 __device__ __forceinline__ void lgkm_wait(int n, half4_t& r, half4_t& q) {
   asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(r), "+v"(q) : "n"(n));
 }
-__device__ __forceinline__ f32x4_t read_f4_untracked(const float* lds) {
-  const uint32_t addr = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
-      (__attribute__((address_space(3))) const float*)(lds)));
-  f32x4_t r;
-  asm volatile("ds_read_b128 %0, %1" : "=v"(r) : "v"(addr));
-  return r;
-}
-__device__ __forceinline__ void lgkm_wait_f4(f32x4_t (&r)[4]) {
-  asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(r[0]), "+v"(r[1]), "+v"(r[2]), "+v"(r[3]));
-}
 // Wait until every LDS (and scalar-memory) operation of the wavefront has returned; the eight
 // registers count as rewritten here, so no copy of them is made before the wait.
 __device__ __forceinline__ void lgkm_wait8(half4_t (&r)[8]) {
@@ -188,26 +166,10 @@ __device__ __forceinline__ void store16(__amdgpu_buffer_rsrc_t r, uint32_t off, 
 }
 
 // One [64][128] tile from global rows base[r * ld + c] (r < rows_valid, else zeros) into `dst`
-// with direct-to-LDS 16-byte loads: block b (rows 4 b .. 4 b + 3) by wavefront b % W.
-template <int W>
-__device__ __forceinline__ void dma_tile(const uint16_t* base, int64_t ld, int rows_valid,
-                                         unsigned char* dst, int wave, int lane) {
-  const __amdgpu_buffer_rsrc_t rsrc = buffer_rsrc(base);
-  const int row_in = lane >> 4, pos = lane & 15;
-#pragma unroll
-  for (int it = 0; it < (kKeys / 4 + W - 1) / W; ++it) {
-    const int b = wave + it * W;
-    if (b >= kKeys / 4) break;
-    const int row = 4 * b + row_in;
-    const int chunk = pos ^ tile_swz(row);
-    const uint32_t off = row < rows_valid ? static_cast<uint32_t>((row * ld + chunk * 8) * 2) : kOob;
-    dma16(rsrc, dst + b * 1024, off);
-  }
-}
-
-// dma_tile with the per-lane part formed once, in one register: the lane's byte offset in block
-// `wave`. Block wave + W * it lies 4 W it rows on (a multiple of 16 for W = 4, so its swizzle is
-// the same), which the load takes as its scalar offset.
+// with direct-to-LDS 16-byte loads: block b (rows 4 b .. 4 b + 3) by wavefront b % W. The per-lane
+// part is one register, the lane's byte offset in block `wave`: block wave + W * it lies 4 W it rows
+// on (a multiple of 16 for W = 4, so its swizzle is the same), which the load takes as its scalar
+// offset.
 struct TileDma {
   static constexpr int W = 4, kPer = kKeys / 4 / W;
   uint32_t off, step;  // step: bytes of 4 W rows (scalar)
@@ -287,7 +249,8 @@ __device__ __forceinline__ int list_pair(int own, int m_max, unsigned pair, int 
 // VALU busy together (a probe's MFMA + exponential loop), and the K / V reads from LDS.
 // Against one workgroup of six or eight wavefronts per CU on 32 query rows (128 KiB of LDS, K
 // operands waited for one by one): 16 rows of 128..512 tokens 36.2 -> 19.9 us, 16 of 1..1024 72.4 ->
-// 39.3, [4096, 3001, 2222, 1531] 187 -> 132 us (543 -> 769 TF/s, 840 in the order of list_pair), config 2's four rows 13.7 -> 13.0.
+// 39.3, [4096, 3001, 2222, 1531] 187 -> 132 us (543 -> 769 TF/s; 827 in the order of list_pair, with the
+// reference maximum as below), config 2's four rows 13.7 -> 13.0.
 // Not kept: the next tile's S^T issued between this one's exponentials and P V (127 against 119 us
 // for 8 rows of 2048: 253 registers, the same clock), s_setprio around the MFMAs (no change).
 // S = 2 where it does not: the longest workgroup's chain of key tiles sets the time (about 1.1 us
@@ -633,9 +596,11 @@ __global__ __launch_bounds__(256) void attn_bwd_dot_kernel(BwdArgs a) {
 // the MFMAs of another, and every operand is read from LDS into the register its last use has just
 // left, waited for with a counted lgkmcnt. The products of a tile's last block therefore still read
 // it while the next tile's scores run: a three-slot ring, one tile ahead.
-// What bounds them: one wavefront per SIMD (364 registers) issues an instruction about every 5
-// cycles, and a 64-row step of dK / dV takes 4440 cycles against 2048 of MFMAs, a 64-key step of dQ
-// 2940 against 1536 (clock stamps); taking the MFMAs out saves only 5%. Against scores,
+// What bounds them: one wavefront per SIMD (364 registers in attn_bwd_kernel; 442 and 30 spilled
+// scalars in attn_bwd_queue_kernel). An unmasked 64-row step of dK / dV is about 600 instructions and
+// takes 4440 cycles against 2048 of MFMAs, a 64-key step of dQ about 460 in 2940 against 1536 (clock
+// stamps); taking the MFMAs out saves only 5%. In dK / dV a block's exponentials all stand beside
+// the MFMAs of the products, none beside those of the scores. Against scores,
 // exponentials and products one after the other with the operands read in batches (465
 // registers): backward of lengths [4096, 3001, 2222, 1531] 610 -> 538 us, of 16 rows of 128..512
 // 100.6 -> 94.6, of config 2's four rows 37.6 -> 35.0.

@@ -155,20 +155,9 @@ def _head_backward(ctx, grad_loss):
     return (grad_hidden.to(torch.float32) * scale).to(ctx.out_dtype)
 
 
-def labelled_first(labelled, n_labelled):
-    """The order that talm_head_order makes, in PyTorch. (dest, src): row r of the input goes to
-    position dest[r] of the labelled-first order and reordered row i is input row src[i]
-    (solution/fused_head.py:290-299; no host sync)."""
-    n = labelled.shape[0]
-    pos = torch.arange(n, device=labelled.device)
-    seen = torch.cumsum(labelled, 0)
-    dest = torch.where(labelled, seen - 1, pos - seen + n_labelled)
-    src = torch.empty_like(dest).index_copy_(0, dest, pos)
-    return dest, src
-
-
 def _order_rows(h16, targets, n_labelled):
-    """(hidden rows, targets) in `labelled_first`'s order and its dest, in one launch."""
+    """(hidden rows, targets) in labelled-first order and dest: row r of the input goes to position
+    dest[r] (solution/fused_head.py:290-299; one launch, no host sync)."""
     if h16.stride(0) < h16.shape[1]:  # expanded or overlapping rows
         h16 = h16.contiguous()
     out = torch.empty(h16.shape, dtype=torch.float16, device=h16.device)

@@ -120,6 +120,15 @@ def test_scale_rows_is_the_reference_arithmetic(n, denom_value):
     assert torch.equal(out.view(torch.int16), expect.view(torch.int16))
 
 
+def _labelled_first(labelled, n_labelled):
+    """(dest, src): row r of the input goes to position dest[r] of the labelled-first order and
+    reordered row i is input row src[i] (solution/fused_head.py:290-299)."""
+    pos = torch.arange(labelled.shape[0])
+    dest = torch.where(labelled, torch.cumsum(labelled, 0) - 1,
+                       pos - torch.cumsum(labelled, 0) + n_labelled)
+    return dest, torch.empty_like(dest).index_copy_(0, dest, pos)
+
+
 @pytest.mark.parametrize("n,hidden,ld", [(1, 8, 8), (8, 1536, 1536), (9, 72, 80), (65, 1544, 1544),
                                          (2048, 1536, 1536), (16385, 64, 64), (140000, 8, 16)])
 def test_head_order_is_labelled_first(n, hidden, ld):
@@ -133,7 +142,7 @@ def test_head_order_is_labelled_first(n, hidden, ld):
     targets = torch.randint(-2, 5, (n,), generator=g)
     labelled = targets >= 0
     count = int(labelled.sum())
-    dest, src = fused_head.labelled_first(labelled, count)
+    dest, src = _labelled_first(labelled, count)
     h = base.cuda()[:, :hidden]
     out, rows_targets, got = fused_head._order_rows(h, targets.cuda(), count)
     assert torch.equal(got.cpu(), dest)
