@@ -69,7 +69,8 @@ struct FwdArgs {
   int64_t v_tok, v_head;
   const int32_t* cu;
   int group;          // query heads per KV head
-  int head_chunks;    // workgroups per KV head (group / heads per workgroup)
+  int wg_heads;       // heads per workgroup, at most H
+  int head_chunks;    // workgroups per KV head (group / wg_heads)
   int list_tiles;     // > 0: the grid is list_pair's list x chunks, its sequences of at most this many tiles
   int n_seqs, chunks;
   int rank_x;         // else the grid's axes: (chunk, sequence, rank), or (rank, chunk, sequence)
@@ -291,8 +292,9 @@ __global__ __launch_bounds__(256 * S, 2) void attn_fwd_kernel(FwdArgs a) {
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wave = wid & 3, grp = wid >> 2;
   const int hh = lane >> 5, l32 = lane & 31;
-  const int head = kvh * a.group + hc * H + wave % H;
+  const int head = kvh * a.group + hc * a.wg_heads + min(wave % H, a.wg_heads - 1);
   const int w0 = q0 + 32 * (wave / H);  // the wavefront's first query row
+  const int row_end = wave % H < a.wg_heads ? len : 0;  // its rows end here (a wavefront without a head: none)
 
   const int qrow = w0 + l32;
   const int qr = min(qrow, len - 1);
@@ -304,7 +306,8 @@ __global__ __launch_bounds__(256 * S, 2) void attn_fwd_kernel(FwdArgs a) {
   }
   const int n_kt = (min(len, q0 + kRows) + kKeys - 1) / kKeys;
   const int n_steps = (n_kt + S - 1) / S;
-  const int my_kt = (min(len, w0 + 32) + kKeys - 1) / kKeys;  // tiles the wavefront's rows see
+  // tiles the wavefront's rows see: none where it has no row
+  const int my_kt = w0 < row_end ? (min(len, w0 + 32) + kKeys - 1) / kKeys : 0;
   const uint16_t* kbase = a.k + static_cast<int64_t>(s0) * a.k_tok + kvh * a.k_head;
   const uint16_t* vbase = a.v + static_cast<int64_t>(s0) * a.v_tok + kvh * a.v_head;
   TileDma kd, vd;
@@ -483,7 +486,7 @@ __global__ __launch_bounds__(256 * S, 2) void attn_fwd_kernel(FwdArgs a) {
       w.y = pack2(o[j][4 * g + 2] * inv, o[j][4 * g + 3] * inv);
       *reinterpret_cast<uint2*>(&os[l32 * kKS + d0]) = w;
     }
-  if (hh == 0 && qrow < len)
+  if (hh == 0 && qrow < row_end)
     a.lse[static_cast<int64_t>(head) * a.n_tokens + s0 + qrow] = (m + __log2f(lsum)) * kLn2;
   // the wavefront reads back its own staging rows: its LDS writes complete first
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -499,7 +502,7 @@ __global__ __launch_bounds__(256 * S, 2) void attn_fwd_kernel(FwdArgs a) {
 #pragma unroll
   for (int it = 0; it < kOut; ++it) {
     const int cc16 = it * 64 + lane, r = cc16 / (kD / 8), cc = cc16 % (kD / 8);
-    store16(ors, w0 + r < len ? static_cast<uint32_t>((r * a.o_tok + 8 * cc) * 2) : kOob, ov[it]);
+    store16(ors, w0 + r < row_end ? static_cast<uint32_t>((r * a.o_tok + 8 * cc) * 2) : kOob, ov[it]);
   }
 }
 
@@ -1277,20 +1280,25 @@ TALM_API int talm_attn_fwd(const uint16_t* q, int64_t q_stride_tok, int64_t q_st
   if (!aligned(q, 16) || !aligned(k, 16) || !aligned(v, 16) || !aligned(out, 16))
     return fail(TALM_EINVAL, "attn_fwd: q, k, v and out must be 16-byte aligned");
   const int group = n_q_heads / n_kv_heads;
-  // query heads per workgroup (4 wavefronts): 4, 2 or 1, what divides the group
-  const int h = group % 4 == 0 ? 4 : group % 2 == 0 ? 2 : 1;
-  const int rows = 32 * (4 / h);
+  // query heads per workgroup (4 wavefronts): 4, 2 or 1, what divides the group; three with an idle
+  // wavefront where a group is a multiple of three and no sequence has more than 64 rows, of which
+  // one head would keep at most two wavefronts busy (12 heads on 4 KV heads, one head / three: 256
+  // rows of 16 tokens 26.8 / 12.9 us, 64 of 33 10.0 / 7.8, 65 of 64 14.6 / 12.9)
+  const bool three = group % 3 == 0 && group % 2 != 0 && max_seqlen <= 64;
+  const int h = three || group % 4 == 0 ? 4 : group % 2 == 0 ? 2 : 1;
+  const int rows = 32 * (4 / h), wg_heads = three ? 3 : h;
   FwdArgs a{};
   a.q = q; a.q_tok = q_stride_tok; a.q_head = q_stride_head;
   a.k = k; a.k_tok = k_stride_tok; a.k_head = k_stride_head;
   a.v = v; a.v_tok = v_stride_tok; a.v_head = v_stride_head;
-  a.cu = cu_seqlens; a.group = group; a.head_chunks = group / h;
+  a.cu = cu_seqlens; a.group = group; a.wg_heads = wg_heads;
+  a.head_chunks = group / wg_heads;
   a.scale_log2 = scale * 1.44269504088896341f;
   a.out = out; a.o_tok = o_stride_tok; a.o_head = o_stride_head;
   a.lse = lse; a.n_tokens = n_tokens;
   // rank-major, so that every sequence's longest workgroups start first; more ranks than a grid's
   // third axis holds go on its first one
-  const unsigned chunks = static_cast<unsigned>(n_q_heads / h), seqs = static_cast<unsigned>(n_seqs);
+  const unsigned chunks = static_cast<unsigned>(n_q_heads / wg_heads), seqs = static_cast<unsigned>(n_seqs);
   const unsigned ranks = static_cast<unsigned>((static_cast<int64_t>(max_seqlen) + rows - 1) / rows);
   a.rank_x = ranks > 65535;
   dim3 grid = a.rank_x ? dim3(ranks, chunks, seqs) : dim3(chunks, seqs, ranks);

@@ -112,6 +112,17 @@ def test_attention_over_head_groups_and_key_splits(lengths, hq, hkv, seed):
     _run(lengths, True, seed, hq, hkv)
 
 
+@pytest.mark.parametrize("lengths,hq,hkv", [
+    ([16, 1, 31, 32], 12, 4), ([33, 64, 0, 63], 9, 1),  # three heads a workgroup: up to 64 rows
+    ([65, 16], 12, 4),                                  # one head a workgroup
+    ([40, 64], 6, 1),                                   # two
+])
+def test_attention_of_short_rows_in_groups_of_three(lengths, hq, hkv):
+    """Workgroups of three heads with a fourth wavefront that has none, against the same reference."""
+    print(f"[case] attention short rows {lengths} heads={hq}/{hkv}", flush=True)
+    _run(lengths, True, 31, hq, hkv)
+
+
 @pytest.mark.parametrize("n,pos", [(256, 64), (256, 200), (600, 70), (600, 255)])
 def test_attention_largest_weight_of_the_first_tiles_is_exact(n, pos):
     """Every score is 0 except key `pos`'s 5 (7.2 in log2 units, below the lazy rescale), and v is 0
