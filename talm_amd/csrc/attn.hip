@@ -1422,13 +1422,18 @@ int attn_bwd_impl(const uint16_t* q, int64_t q_stride_tok, int64_t q_stride_head
   a.dv = dv; a.dv_tok = dv_stride_tok; a.dv_head = dv_stride_head;
   a.cos = rope ? cos : nullptr; a.sin = rope ? sin : nullptr; a.cs_tok = cs_stride;
   // The queue for more than two items per CU (what there is to balance), up to one sequence per lane,
-  // where its indices fit 32 bits. Backward, grid / queue: [1500, 800] with 14 / 2 heads (532 items)
+  // where its indices fit 32 bits, and unless the items are all short (one tile per sequence, at most
+  // 96 of its 128 rows on the average). Backward, grid / queue: [1500, 800] with 14 / 2 heads (532 items)
   // 78 / 72 us, eight rows of 128..512 (672) 59 / 51, [3000] (576) 137 / 134, but [2048] (384) 82.3
-  // / 84.2, four rows of 128..512 (312) 34.9 / 35.9: finding and drawing an item costs 1-2 us.
+  // / 84.2, four rows of 128..512 (312) 34.9 / 35.9: finding and drawing an item costs 1-2 us. One
+  // tile per sequence, 64 sequences of 33, 64, 96 and 128 tokens with 12 / 2 heads (1536): 46.3 / 52.8,
+  // 60.2 / 61.3, 86.2 / 82.6, 105 / 94; 24 sequences, 16 / 16 heads (768): 31.9 / 35.0, 37.5 / 40.6,
+  // 51.3 / 53.8, 60.5 / 60.6.
   const int64_t items = 2 * static_cast<int64_t>(n_q_heads) *
                         std::min<int64_t>(n_tokens / (32 * W) + n_seqs, static_cast<int64_t>(n_seqs) * a.n_tiles);
   a.n_seqs = n_seqs;
-  if (n_seqs <= kListSeqs && items > 2 * device_cus() && items < (int64_t{1} << 30) &&
+  if (n_seqs <= kListSeqs && items > 2 * device_cus() &&
+      (a.n_tiles > 1 || n_tokens > 96 * static_cast<int64_t>(n_seqs)) && items < (int64_t{1} << 30) &&
       workspace_bytes >= need + kQueueBytes) {
     a.counter = reinterpret_cast<unsigned*>(a.dv_part + n_tokens * n_q_heads * kD);
     a.queue_wgs = static_cast<unsigned>(std::min<int64_t>(items, device_cus()));

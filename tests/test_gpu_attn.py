@@ -208,6 +208,8 @@ def test_attention_backward_with_the_rotary_backward_folded_in(lengths, seed):
     ([7 * i % 300 for i in range(64)], 12, 2),         # one sequence per lane
     ([7 * i % 300 for i in range(65)], 12, 2),         # one more: no queue
     ([2305], 16, 8),                                   # 608 items: just above two per CU of 256
+    ([96] * 31 + [97], 12, 2),                         # one tile each, 96 rows on the average or more
+    ([96] * 32, 12, 2),                                # not more: no queue
 ])
 def test_attention_backward_from_the_queue(lengths, hq, hkv):
     """The same workgroups' work whether drawn from the queue or launched one by one (a workspace
