@@ -803,13 +803,20 @@ void launch_tiles(QkvArgs& a, hipStream_t stream) {
 template <bool kDown>
 void launch_proj(QkvArgs& a, hipStream_t stream) {
   a.cs_vec = a.cos && aligned(a.cos, 16) && aligned(a.sin, 16) && a.cs_stride % 4 == 0;
-  // 128-row tiles once the 64-row ones exceed one round at two workgroups per CU. Measured, 64 / 128
-  // rows: forward at 3000 tokens 46.5 / 36.6 us, at 5015 73.0 / 68.8, input gradient 41.3 / 31.9 and 54.7 /
-  // 39.2; at 2048 tokens and below (one round of 64-row tiles) half as many workgroups would run. A
-  // tile's rows of x and of the extra step's operand must lie within 32-bit offsets.
-  const int64_t small = static_cast<int64_t>((a.n_tokens + QkvShape::kBM - 1) / QkvShape::kBM) *
-                        ((a.n_out + QkvShape::kBN - 1) / QkvShape::kBN);
-  if (small > 2 * device_cus() && fits32(QkvWide::kBM, a.ldx) &&
+  // 128-row tiles once the 64-row ones exceed one round at two workgroups per CU, where a CU's share
+  // of them takes no longer: a 128-row tile's work is that of two 64-row ones in about 3/4 of the time.
+  // Measured, 64 / 128 rows: forward (hidden 1536 to 2048) at 3000 tokens (3 / 2 tiles per CU) 46.5 /
+  // 36.6 us, at 5015 (5 / 3) 73.0 / 68.8, input gradient 41.3 / 31.9 and 54.7 / 39.2; but 4096 to 6144 at
+  // 1312 tokens (4 / 3: 528 tiles of 128 rows, just past a round) 100 / 115; at 2048 tokens and below
+  // (one round of 64-row tiles) half as many workgroups would run. A tile's rows of x and of the
+  // extra step's operand must lie within 32-bit offsets.
+  const auto tiles = [&](int rows) {
+    return static_cast<int64_t>((a.n_tokens + rows - 1) / rows) *
+           ((a.n_out + QkvShape::kBN - 1) / QkvShape::kBN);
+  };
+  const int64_t cus = device_cus(), small = tiles(QkvShape::kBM);
+  const int64_t per_cu = (small + cus - 1) / cus, wide_per_cu = (tiles(QkvWide::kBM) + cus - 1) / cus;
+  if (small > 2 * cus && 3 * wide_per_cu <= 2 * per_cu && fits32(QkvWide::kBM, a.ldx) &&
       (kDown || fits32(QkvWide::kBM, a.ldt)))
     launch_tiles<QkvWide, kDown>(a, stream);
   else

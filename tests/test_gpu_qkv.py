@@ -173,6 +173,11 @@ def test_projections_on_128_row_tiles(n):
     test_qkv_lora_bwd_dx_matches_fp32(n, 2048, 256, 32)
 
 
+def test_projection_of_two_rounds_on_64_row_tiles():
+    """21 x 48 tiles of 64 rows, four per CU of 256, where 11 x 48 of 128 rows would be three."""
+    test_qkv_lora_fwd_down_matches_fp32(1312, 64, 6144, [(0, 4096), (5120, 6144)], 5120, False)
+
+
 def test_extra_step_with_a_wide_row_stride():
     """128 rows of u 2^23 + 2^17 columns apart: 64-row tiles reach them with 32-bit offsets, 128-row
     ones would not (516 tiles of 64 x 128, more than a round). The same bits as of contiguous rows."""
